@@ -294,6 +294,83 @@ def test_qkv_proj_unstaged_v_matches_inorder_kernel(cuda, dtype, gemm_variant):
     assert float((qk.float() - ref[:, : 2 * d]).abs().max()) < 0.05
 
 
+# gemm_ring_kernel's tile configurations (TX_GEMM_VARIANT 1000 ..) against the
+# in-order kernel, bit for bit: one to five K steps (fewer than the ring's
+# stages, equal, more), one tile and a ragged last tile in M and N, N % 8 == 4
+# (the direct epilogue), fp32 results and hi/lo pairs.
+RING_SHAPES = [(1, 8, 64), (64, 64, 256), (65, 196, 128), (129, 200, 192), (300, 584, 320), (1000, 1032, 512)]
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m,n,k", RING_SHAPES)
+def test_gemm_ring_configurations_match_inorder_kernel(cuda, dtype, m, n, k, gemm_variant):
+    log(f"gemm ring {m}x{n}x{k} {dtype}")
+    a = _randn((m, k), dtype, cuda, 71)
+    w = _randn((n, k), dtype, cuda, 72, 0.02)
+    bias = _randn((n,), dtype, cuda, 73, 0.1)
+    x = _randn((m, n), dtype, cuda, 74)
+    x32 = _randn((m, n), torch.float32, cuda, 75)
+    rows = (torch.arange(m, device=cuda) % 7 != 3).to(torch.uint8)
+
+    def run_all():
+        outs = [_C.gemm(a, w), _C.gemm(a, w, bias, gelu=True), _C.gemm(a, w, bias, gelu=True, split_out=True),
+                _C.gemm(a, w, bias, residual=x32, out_dtype=torch.float32, row_valid=rows, mask_out=True)]
+        for kw in ({"mask_delta": True}, {"mask_out": True}):
+            c = x.clone()
+            outs.append(_C.gemm(a, w, bias, residual=c, out=c, row_valid=rows, **kw))
+        return outs
+
+    gemm_variant(0)
+    ref = run_all()
+    for v in [*range(1000, 1006), -1]:
+        gemm_variant(v)
+        for i, (r, g) in enumerate(zip(ref, run_all())):
+            assert torch.equal(g, r), f"variant {v} output {i}"
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("m,n,k", [(17, 72, 2048), (64, 512, 2176), (200, 1024, 2048), (256, 4096, 2048)])
+def test_gemm_ring_four_sum_order(cuda, dtype, m, n, k, gemm_variant):
+    """M <= 256, K >= 2048: the ring tiles add K in the order of the 16x16
+    kernel's four waves (variant 10), bit for bit."""
+    log(f"gemm ring four sums {m}x{n}x{k} {dtype}")
+    a = _randn((m, k), dtype, cuda, 76)
+    w = _randn((n, k), dtype, cuda, 77, 0.02)
+    bias = _randn((n,), dtype, cuda, 78, 0.1)
+    x = _randn((m, n), torch.float32, cuda, 79)
+    got = {}
+    for v in (10, 1000, 1001, -1):
+        gemm_variant(v)
+        got[v] = (_C.gemm(a, w, bias, gelu=True), _C.gemm(a, w, bias, residual=x, out_dtype=torch.float32))
+    for v in (1000, 1001, -1):
+        assert all(torch.equal(p, q) for p, q in zip(got[10], got[v])), f"variant {v}"
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("b,s,d,h", [(1, 64, 64, 1), (3, 100, 256, 4), (5, 129, 320, 5), (2, 421, 192, 3),
+                                     (9, 40, 256, 2), (1, 1023, 128, 1)])
+def test_qkv_proj_ring_configurations(cuda, dtype, b, s, d, h, gemm_variant):
+    """Packed Q/K/V through every ring tile: tiles that hold k and V columns,
+    V^T runs that start and end inside an eight-position chunk, two sequences
+    in a tile, and sequences shorter than a tile (written unstaged).  The
+    columns of V^T past the sequence stay as they were."""
+    log(f"qkv ring b{b} s{s} d{d} {dtype}")
+    x = _randn((b * s, d), dtype, cuda, 81)
+    w = _randn((3 * d, d), dtype, cuda, 82, 0.02)
+    bias = _randn((3 * d,), dtype, cuda, 83, 0.1)
+
+    def run():
+        vt = torch.full((b, h, d // h, _C.vt_ld(s)), 7.0, dtype=dtype, device=cuda)
+        return _C.qkv_proj(x, w, bias, b, s, h, vt=vt)
+
+    gemm_variant(0)
+    qk0, vt0 = run()
+    for v in [*range(1000, 1006), -1]:
+        gemm_variant(v)
+        qk, vt = run()
+        assert torch.equal(qk, qk0) and torch.equal(vt, vt0), f"variant {v}"
+
+
 def test_gemm_wide_row_stride_takes_64bit_kernel(cuda):
     """lda past the 256-row kernel's 32-bit DMA offsets ((255 lda + 56) * 2 >
     2^31 - 1) routes to the 64-bit-addressed 128x128 kernel: the product of

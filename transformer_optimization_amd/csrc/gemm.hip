@@ -24,6 +24,7 @@
 #include <cstdlib>
 
 #include "common.hpp"
+#include "gemm_common.hpp"
 #include "tx_internal.hpp"
 
 namespace tx {
@@ -34,23 +35,6 @@ constexpr int GEMM_BK = 64;
 // the odd rows of any 16-row group, so 8-lane (128 B) and 16-lane (256 B)
 // access phases are both conflict-free.
 __device__ __forceinline__ int gemm_swz(int r) { return (r & 7) ^ ((r >> 3) & 1); }
-
-// Workgroup -> tile mapping.  Workgroups are dispatched round-robin over the
-// 8 XCDs (workgroup i runs on XCD i % 8); remap so that each XCD receives a
-// contiguous range of logical tiles, then walk tiles in groups of GROUP tile
-// rows so that concurrently running tiles share A rows and W columns in L2.
-__device__ __forceinline__ void gemm_tile_of(int pid, int nwg, int tiles_m, int tiles_n,
-                                             int& tm, int& tn, int GROUP = 8) {
-  const int x = pid & 7, i = pid >> 3, q = nwg >> 3, r = nwg & 7;
-  pid = x * q + (x < r ? x : r) + i;
-  const int width = GROUP * tiles_n;
-  const int group = pid / width;
-  const int first_m = group * GROUP;
-  const int gsz = (tiles_m - first_m) < GROUP ? (tiles_m - first_m) : GROUP;
-  const int in_group = pid - group * width;
-  tm = first_m + in_group % gsz;
-  tn = in_group / gsz;
-}
 
 template <typename T, typename TC, typename TB, typename TR, int BM, int BN, int WM, int WN, bool QKV>
 __global__ __launch_bounds__(WM* WN * 64) void gemm_kernel(GemmArgs g) {
@@ -246,66 +230,6 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_kernel(GemmArgs g) {
   }
 }
 
-// ------------------------------------------------------ shared epilogue
-// Epilogue of four consecutive output columns n..n+3 of row m (the D^T
-// accumulator layout: lane holds columns, not rows).  acc: the fp32 sums;
-// bv: the bias values (0 without BIAS); rv: the residual values (read before
-// any store of the group, since the residual may alias C); valid: the row's
-// row_valid flag (true without masks).
-__device__ __forceinline__ bool gemm_row_valid(const GemmArgs& g, int m) {
-  const bool need = (g.epi & (TX_EPI_MASK_DELTA | TX_EPI_MASK_OUT)) && g.row_valid != nullptr;
-  return !need || g.row_valid[m] != 0;
-}
-template <typename TC, bool QKV>
-__device__ __forceinline__ void gemm_finish4(const GemmArgs& g, int m, int n, const float* acc,
-                                             const float* bv, const float* rv, bool valid) {
-  const uint32_t epi = g.epi;
-  TC* __restrict__ C = (TC*)g.c;
-  if (!QKV && (epi & TX_EPI_SPLIT_OUT)) {
-    // fp32-residual policy: the unrounded value as a hi/lo pair.
-    float hi[4], lo[4];
-#pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      float t = acc[e] + bv[e];
-      if (epi & TX_EPI_GELU_ERF) t = gelu_erf(t);
-      hi[e] = round_to<TC>(t);
-      lo[e] = t - hi[e];
-    }
-    store4<TC>(C + (int64_t)m * g.ldc + n, hi);
-    store4<TC>(C + (int64_t)m * g.ldc + n + g.n, lo);
-    return;
-  }
-  float v[4];
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    float t = round_to<TC>(acc[e] + bv[e]);
-    if (epi & TX_EPI_GELU_ERF) t = round_to<TC>(gelu_erf(t));
-    v[e] = t;
-  }
-  if (!QKV) {
-    if (epi & TX_EPI_RESIDUAL) {
-      const bool drop = (epi & TX_EPI_MASK_DELTA) && !valid;
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = round_to<TC>(rv[e] + (drop ? 0.f : v[e]));
-    }
-    if ((epi & TX_EPI_MASK_OUT) && !valid) {
-#pragma unroll
-      for (int e = 0; e < 4; ++e) v[e] = 0.f;
-    }
-  }
-  if (!QKV || n < g.qk_cols) {
-    store4<TC>(C + (int64_t)m * g.ldc + n, v);
-  } else {
-    // V columns go head-transposed into vt[b][h][d][s].
-    const int nv = n - g.qk_cols;
-    const int hh = nv / g.head_dim, d0 = nv - hh * g.head_dim;
-    const int b = m / g.seq, sq = m - b * g.seq;
-    TC* dst = (TC*)g.vt + ((int64_t)(b * g.heads + hh) * g.head_dim + d0) * g.ldvt + sq;
-#pragma unroll
-    for (int e = 0; e < 4; ++e) dst[(int64_t)e * g.ldvt] = from_f32<TC>(v[e]);
-  }
-}
-
 // ================================================================ big tiles
 // gemm_big_kernel: 128 x 128 / 256 x 256 tiles, compiler-scheduled; the
 // baseline gemm_hp_kernel is measured against (TX_GEMM_VARIANT 20 / 19).
@@ -337,21 +261,6 @@ __device__ __forceinline__ void gemm_finish4(const GemmArgs& g, int m, int n, co
 // read the fragments of the next k16 group while the MFMAs of this one run.
 // The defaults use bits 1 and 2 (the priority raise is a scheduling fence
 // that keeps the compiler from hoisting the fragment reads).
-template <int CH>
-__device__ __forceinline__ int big_swz(int r) {
-  // CH = 16-byte chunks per LDS row.  16 consecutive rows read at one
-  // logical chunk must cover all 64 banks.  A ds_read_b128 serves 16 lanes
-  // per cycle from 64 four-byte banks, and the bank group of a 16-byte unit
-  // (measured with SQ_LDS_BANK_CONFLICT on gfx950 over seven access
-  // patterns) is address bits 4..7 with bit 10 folded into bit 4: with
-  // 128-byte rows, rows r and r + 8 already differ in that bit, so the row's
-  // low three bits are the whole swizzle.  Also folding in bit 3 of the row
-  // cancels the hardware's term and pairs rows r and r + 8 (two cycles per
-  // read instead of one).
-  if constexpr (CH == 8) return r & 7;
-  else return (r >> 2) & 3;
-}
-
 // Workgroups of one tile shape resident per CU, bounded by its LDS ring
 // (160 KB per CU); the register budget (the launch bound's minimum waves per
 // SIMD) is sized to keep that many resident.
@@ -1243,6 +1152,10 @@ static int launch_big(const GemmArgs& g, hipStream_t st) {
   return hipGetLastError() == hipSuccess ? TX_OK : TX_EHIP;
 }
 
+template <typename T> constexpr int dt_code() {
+  return std::is_same<T, float>::value ? TX_F32 : std::is_same<T, f16>::value ? TX_F16 : TX_BF16;
+}
+
 static inline bool al(const void* p, int bytes) { return ((uintptr_t)p % bytes) == 0; }
 
 template <typename T, typename TC, typename TB, typename TR, int BN, bool QKV, int NS = 2>
@@ -1299,6 +1212,16 @@ static int hp_width(const GemmArgs& g, int cus) {
   return best;
 }
 
+// Modelled time (us) of gemm_hp_kernel at a tile width: c + rounds (a k + e),
+// fitted to the same 170 random shapes as gemm_ring_kernel's configurations
+// (standard error 12-13%).
+static double hp_model_us(const GemmArgs& g, int cus, int bn) {
+  const int i = bn == 256 ? 0 : bn == 192 ? 1 : 2;
+  static const double c[3] = {0.0, 0.0, 0.836}, a[3] = {0.0212, 0.0169, 0.0117}, e[3] = {12.1, 10.3, 7.32};
+  const long tiles = (long)((g.m + 255) / 256) * ((g.n + bn - 1) / bn);
+  const long rounds = (tiles + cus - 1) / cus;
+  return c[i] + (double)rounds * (a[i] * g.k + e[i]);
+}
 
 template <typename T, typename TC, typename TB, typename TR, bool QKV>
 static int launch_gemm_typed(const GemmArgs& g0, hipStream_t st) {
@@ -1337,6 +1260,26 @@ static int launch_gemm_typed(const GemmArgs& g0, hipStream_t st) {
   // The library splits K over four waves at small M and K >= 2048 (NW = 4
   // reproduces that order); everywhere else it accumulates in order.
   const bool lsu4 = g.k >= 2048 && g.k % 128 == 0;
+  // gemm_ring_kernel: K a multiple of 64 (64-bit row strides excluded).
+  const bool ring_ok = vec_ok && g.k % 64 == 0 && hp_offsets_fit(g.lda, g.ldw, g.k, sizeof(T));
+  auto ring = [&](int cfg, bool ks4) {
+    return launch_gemm_ring(g, dt_code<T>(), dt_code<TC>(), dt_code<TR>(), QKV, cfg, ks4, st);
+  };
+  double ring_us = 0.0;
+  const bool ring_ks4 = skinny_ok && lsu4;
+  const int ring_cfg = ring_pick(g.m, g.n, g.k, cus, ring_ks4, &ring_us);
+  if (variant >= 1000 && variant < 1006 && ring_ok) return ring(variant - 1000, ring_ks4 && variant < 1002);
+  // Small M: 16 x 16 blocks while they are few (c2's shapes: 64x1536x512 4.9
+  // against 5.3 us), ring tiles (same bits) where the blocks' operand reads
+  // grow past them (190x2048x2048 25.3 against 10.6 us, 102x3072x1024 14.2
+  // against 8.2).  Modelled times in us, fitted to 60 random shapes with
+  // M 17 .. 256 (within 10%): a base, the chain over K, and the operand reads
+  // of all blocks.
+  if (skinny_ok && ring_ok && variant < 0) {
+    const double reads = (double)((g.m + 15) / 16) * ((g.n + 15) / 16) * g.k;
+    const double lsu_us = lsu4 ? 4.06 + 2.67e-4 * g.k + 6.4e-6 * reads : 2.98 + 8.07e-4 * g.k + 6.8e-6 * reads;
+    if (ring_us < lsu_us) return ring(ring_cfg, ring_ks4);
+  }
   if (skinny_ok && g.k % 32 == 0 && ((variant < 0 && !lsu4) || variant == 11)) {
     const long blocks = (long)((g.m + 15) / 16) * ((g.n + 15) / 16);
     gemm_lsu_kernel<T, TC, TB, TR, QKV, 1><<<dim3((unsigned)blocks), dim3(64), 0, st>>>(g);
@@ -1358,23 +1301,29 @@ static int launch_gemm_typed(const GemmArgs& g0, hipStream_t st) {
   }
   const bool big_ok = g.k % 64 == 0 && g.m >= 256 && vec_ok;
   if (!big_ok || variant == 0) return launch_gemm_small<T, TC, TB, TR, QKV>(g, st);
-  // Otherwise fp32 C (the fp32-residual policy's out_proj / FFN-out sums)
-  // with short K keeps the 128x128 kernel: gemm_hp_kernel's staged epilogue
-  // covers 16-bit C only, and with its direct fp32 epilogue the 256-wide
-  // tiles took 471 vs 374 us at c5's out_proj (K = 1024); c5's FFN-out
-  // (K = 8192) is faster on them (1768 vs 2020 us).
+  // fp32 C with short K: gemm_hp_kernel's staged epilogue covers 16-bit C
+  // only, and its direct fp32 epilogue on 256-wide tiles took 471 us at
+  // 100000x1024x1024, where ring tiles take 360.
   // Tall operands (M >= 32768, so A streams from HBM rather than staying in
-  // the caches) with a short K panel (K <= 2048) take 128-wide tiles: their
-  // third K stage covers the longer latency.  c5 (M = 100000), launches
-  // repeated in isolation: QKV 767 -> 689 us, FFN-in 2274 -> 2022 us, the
-  // fp32-output out_proj 382 -> 351 us (against the 128x128 two-stage
-  // kernel); FFN-out (K = 8192) stays 256-wide (1646 vs 1732 us).
+  // the caches) with a short K panel (K <= 2048): of the 256-row tiles the
+  // 128-wide ones, whose third K stage covers the longer latency; ring tiles
+  // of 128 x 192 where the model prefers them (100000 rows: QKV 663 -> 612
+  // us, FFN-in 1058 -> 971).
   const bool tall = g.m >= 32768 && g.k <= 2048;
   if (variant < 0) {
-    if (tall)
-      variant = 128;
-    else
-      variant = (sizeof(TC) == 4 && !(g.epi & TX_EPI_SPLIT_OUT) && g.k < 4096) ? 20 : hp_width(g, cus);
+    double hp_us = 0.0;
+    const bool big128 = !tall && sizeof(TC) == 4 && !(g.epi & TX_EPI_SPLIT_OUT) && g.k < 4096;
+    variant = tall ? 128 : hp_width(g, cus);
+    hp_us = hp_model_us(g, cus, variant);
+    // gemm_hp_kernel writes V^T element by element when a 16-row chunk can
+    // span two sequences; gemm_ring_kernel does not (S = 421, 2105x3072x1024:
+    // 24.3 against 21.2 us, where the model has 20.1 and 20.9).
+    if (QKV && g.seq % 16 != 0) hp_us *= 1.2;
+    if (big128) variant = 20;
+    // Smaller tiles where their modelled time is less (ring_pick), and for
+    // all fp32 results that took the 128x128 kernel (16000x1024x1024 53 to 55
+    // against 56 us, 5003x1024x1024 20 against 26 us).
+    if (ring_ok && (big128 || ring_us < hp_us)) return ring(ring_cfg, false);
   }
   // gemm_hp_kernel's per-lane DMA offsets are 32-bit (hp_offsets_fit); wider
   // row strides take the 128x128 kernel, which addresses in 64 bits.
