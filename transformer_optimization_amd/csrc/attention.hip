@@ -88,6 +88,17 @@ __device__ __forceinline__ int ax_tile_swz(int key) {
 __device__ __forceinline__ void ax_work_of(int nq, int causal, int& bh, int& qb) {
   int pid = blockIdx.x;
   const int nwg = gridDim.x;
+  const int heads8 = nwg / nq;  // (batch, head) pairs, 8 * hx when the branch is taken
+  if (causal && (heads8 & 7) == 0) {
+    // Whole heads per XCD: its workgroups start with the longest rows of all
+    // its heads, so that the short ones fill the CUs that end first (head by
+    // head, the last head's longest rows started last: 32 x 8 heads of 512
+    // keys 96.9 -> 67.6 us, 16 heads of 5003, online 96.0 -> 84.8).
+    const int hx = heads8 >> 3, i = pid >> 3, r = i / hx;
+    bh = (pid & 7) * hx + (i - r * hx);
+    qb = nq - 1 - r;
+    return;
+  }
   const int x = pid & 7, i = pid >> 3, q = nwg >> 3, r = nwg & 7;
   pid = x * q + (x < r ? x : r) + i;
   bh = pid / nq;
