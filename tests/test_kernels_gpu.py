@@ -834,6 +834,55 @@ def test_online_softmax_running_max_rebase(cuda, pattern, dtype, hd):
     assert err <= 4 * 2.0 ** -8 * max(exact.abs().max().item(), 1e-3)
 
 
+@pytest.fixture
+def flash_groups():
+    import os
+    old = os.environ.get("TX_ATTN_FLASH")
+    yield lambda n: os.environ.__setitem__("TX_ATTN_FLASH", str(n))
+    if old is None:
+        os.environ.pop("TX_ATTN_FLASH", None)
+    else:
+        os.environ["TX_ATTN_FLASH"] = old
+
+
+@pytest.mark.parametrize("dtype,hd", [(torch.bfloat16, 64), (torch.float16, 64), (torch.bfloat16, 128)])
+@pytest.mark.parametrize("b,h,s,causal,masked", [(1, 2, 1, False, False), (2, 4, 63, True, False),
+                                                 (1, 3, 65, True, True), (2, 2, 128, False, True),
+                                                 (2, 8, 333, True, False), (1, 4, 449, False, True)])
+def test_online_softmax_key_groups(cuda, dtype, hd, b, h, s, causal, masked, flash_groups):
+    """One and two key groups per workgroup, both V layouts: rows whose second
+    group has no tile or no admissible key, odd and even tile counts, a fully
+    masked sequence (its rows are 0).  Against fp32 attention: q is rounded
+    once more (scaled into log2 units) and p once, 2^-p relative each, so 2^-p
+    times a few row magnitudes bounds the difference."""
+    log(f"online groups b{b} h{h} s{s} hd{hd} causal={causal} masked={masked} {dtype}")
+    qkv = _randn((b, s, 3 * h * hd), dtype, cuda, 171, 0.8)
+    q, k, v = (qkv[..., j * h * hd:(j + 1) * h * hd].view(b, s, h, hd).transpose(1, 2) for j in range(3))
+    valid = None
+    if masked:
+        valid = torch.rand((b, s), generator=_gen(172)).to(cuda) < 0.6
+        valid[-1] = False
+    sc = (q.float() @ k.float().transpose(2, 3).contiguous()) * hd ** -0.5
+    if causal:
+        sc = sc.masked_fill(torch.ones((s, s), dtype=torch.bool, device=cuda).triu(1), float("-inf"))
+    if masked:
+        sc = sc.masked_fill(~valid[:, None, None, :], float("-inf"))
+    ref = torch.softmax(sc, -1).nan_to_num(0.0) @ v.float()
+    qk = qkv[..., :2 * h * hd].reshape(b * s, 2 * h * hd).contiguous()
+    vt = torch.zeros((b, h, hd, _C.vt_ld(s)), dtype=dtype, device=cuda)
+    vt[..., :s] = v.transpose(2, 3)
+    eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    for n in (1, 2):
+        flash_groups(n)
+        o1 = _C.flash_attn(qk, vt, b, s, h, hd, hd ** -0.5, causal, key_valid=valid, softmax="online")
+        o2 = _C.flash_attn_strided(q, k, v, hd ** -0.5, causal, key_valid=valid, softmax="online")
+        for o in (o1.view(b, s, h, hd).transpose(1, 2), o2):
+            err = (o.float() - ref).abs().amax()
+            assert float(err) <= 8 * eps * float(v.float().abs().amax()), f"{n} groups: {float(err)}"
+            if masked:
+                assert not o[-1].any()
+
+
 @pytest.mark.parametrize("s,hd,causal", [(96, 64, False), (40, 64, False), (17, 64, True), (1500, 64, True),
                                           (2048, 128, False), (1100, 128, True)])
 def test_fully_masked_rows_are_zero_not_nan(cuda, s, hd, causal):
