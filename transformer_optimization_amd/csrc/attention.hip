@@ -395,66 +395,116 @@ __device__ __forceinline__ void ax_round2(float& a, float& b) {
   }
 }
 
-// The 32 eager scores of this lane for one tile, as fp32 values of T:
-// round(acc), then for a non-power-of-two scale round(round(acc) * scale).
-// (For a power-of-two scale the product is exact and formed in ax_shift.)
-template <typename T, bool EXACT_SCALE, int NT = 2>
-__device__ __forceinline__ void ax_round_scores(f32x16* s, float scale) {
+// The eager scores of NT 32-key halves of a tile (16 a lane each), rounded as
+// eager rounds them: round(acc), then round(round(acc) * scale).
+//   bf16: fp32 registers holding bf16 values (one conversion each).  EXACT (a
+//     power-of-two scale): the product is exact and formed with the
+//     subtraction of the row max in one fma.
+//   fp16: packed pairs, so that a score takes two instructions up to its
+//     shifted value instead of six.  EXACT (the scale is an fp16 value, 1/8 at
+//     head dim 64): the product of two fp16 values is exact in fp32, so
+//     v_pk_mul_f16 rounds it as eager's fp32 multiply and conversion do,
+//     subnormal results included.  Otherwise the multiply runs in fp32 straight
+//     from the packed half (v_fma_mix_f32).  The shift reads the packed half
+//     too: fma(s, 1, -m) = s - m.
+template <typename T, bool EXACT, int NT = 2>
+struct AxScores;
+template <bool EXACT, int NT>
+struct AxScores<bf16, EXACT, NT> {
+  static constexpr bool FUSED = EXACT;  // the scale is still to be applied
+  float v[NT][16];
+  __device__ __forceinline__ void round(const f32x16* acc, float scale) {
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
+    for (int t = 0; t < NT; ++t) {
 #pragma unroll
-    for (int r = 0; r < 16; r += 2) {
-      float a = s[t][r], b = s[t][r + 1];
-      ax_round2<T, false>(a, b);
-      if (!EXACT_SCALE) {
-        a *= scale;
-        b *= scale;
-        ax_round2<T>(a, b);
+      for (int r = 0; r < 16; r += 2) {
+        float a = acc[t][r], b = acc[t][r + 1];
+        ax_round2<bf16, false>(a, b);
+        if (!EXACT) {
+          a *= scale;
+          b *= scale;
+          ax_round2<bf16>(a, b);
+        }
+        v[t][r] = a;
+        v[t][r + 1] = b;
       }
-      s[t][r] = a;
-      s[t][r + 1] = b;
     }
   }
+  __device__ __forceinline__ float shift(int t, int r, float scale, float m) const {
+    return EXACT ? __builtin_fmaf(v[t][r], scale, -m) : v[t][r] - m;
+  }
+};
+template <bool EXACT, int NT>
+struct AxScores<f16, EXACT, NT> {
+  static constexpr bool FUSED = false;
+  uint32_t h[NT][8];
+  __device__ __forceinline__ void round(const f32x16* acc, float scale) {
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    const h2 sc = {(_Float16)scale, (_Float16)scale};
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const uint32_t w = pack2_raw<f16>(acc[t][2 * i], acc[t][2 * i + 1]);
+        if constexpr (EXACT) {
+          h[t][i] = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, w) * sc);
+        } else {
+          float lo, hi;
+          asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel_hi:[1,0,0]" : "=v"(lo) : "v"(w), "v"(scale));
+          asm("v_fma_mix_f32 %0, %1, %2, 0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(hi) : "v"(w), "v"(scale));
+          h[t][i] = pack2_raw<f16>(lo, hi);
+        }
+      }
+    }
+  }
+  __device__ __forceinline__ float shift(int t, int r, float, float m) const {
+    float x;
+    if (r & 1)
+      asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(x) : "v"(h[t][r >> 1]), "v"(m));
+    else
+      asm("v_fma_mix_f32 %0, %1, 1.0, -%2 op_sel_hi:[1,0,0]" : "=v"(x) : "v"(h[t][r >> 1]), "v"(m));
+    return x;
+  }
+};
+
+// The row max that eager subtracts, from the largest raw accumulator (max
+// commutes with the monotone rounding and scaling).
+template <typename T, bool EXACT>
+__device__ __forceinline__ float ax_row_max(float mx, float scale) {
+  float hi = mx, unused = 0.f;
+  ax_round2<T>(hi, unused);
+  hi *= scale;
+  if constexpr (!AxScores<T, EXACT, 1>::FUSED) ax_round2<T>(hi, unused);
+  return hi;
 }
 
-// Masked keys (invalid, past S, or after the query when causal) -> -inf.
+// Masked keys (invalid, past S, or after the query when causal) -> val (-inf
+// for scores, 0 for exponentials already formed).
 // PERM: the scores come from the key-permuted K operand (AxKOff::init_perm).
-template <bool PERM = false>
-__device__ __forceinline__ void ax_mask(float (*x)[16], uint64_t kmask, int causal, int kt0, int myq,
-                                        int lane) {
-  const float NEG_INF = -__builtin_inff();
-  // Key of slot (t, r) = kt0 + h4 + c with a compile-time c; shift the mask
-  // and the causal limit by the lane's part h4 once.
-  const int h4 = (lane >> 5) << (PERM ? 3 : 2);
-  const uint64_t km = kmask >> h4;
-  const int lim = causal ? myq - kt0 - h4 : AX_BN;
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-#pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int c = PERM ? 32 * t + ((r >> 3) << 4) + (r & 7) : 32 * t + ((r >> 2) << 3) + (r & 3);
-      const bool ok = ((km >> c) & 1ull) && c <= lim;
-      x[t][r] = ok ? x[t][r] : NEG_INF;
-    }
-  }
-}
-
-// Same with a chosen replacement value (0 for exponentials already formed).
 template <bool PERM = false>
 __device__ __forceinline__ void ax_mask_to(float (*x)[16], uint64_t kmask, int causal, int kt0, int myq,
                                            int lane, float val) {
+  // Key of slot (t, r) = kt0 + h4 + c with a compile-time c; shift the mask
+  // and the causal limit by the lane's part h4 once.
   const int h4 = (lane >> 5) << (PERM ? 3 : 2);
-  const uint64_t km = kmask >> h4;
   const int lim = causal ? myq - kt0 - h4 : AX_BN;
+  // Key mask and causal limit as one bit per key.
+  uint64_t km = kmask >> h4;
+  if (lim < 0) km = 0;
+  else if (lim < 63) km &= (2ull << lim) - 1;
 #pragma unroll
   for (int t = 0; t < 2; ++t) {
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
       const int c = PERM ? 32 * t + ((r >> 3) << 4) + (r & 7) : 32 * t + ((r >> 2) << 3) + (r & 3);
-      const bool ok = ((km >> c) & 1ull) && c <= lim;
-      x[t][r] = ok ? x[t][r] : val;
+      x[t][r] = ((km >> c) & 1ull) ? x[t][r] : val;
     }
   }
+}
+template <bool PERM = false>
+__device__ __forceinline__ void ax_mask(float (*x)[16], uint64_t kmask, int causal, int kt0, int myq,
+                                        int lane) {
+  ax_mask_to<PERM>(x, kmask, causal, kt0, myq, lane, -__builtin_inff());
 }
 
 // ax_mask (or ax_mask_to, with val) for the 16 scores of one 32-key half t
@@ -463,14 +513,12 @@ __device__ __forceinline__ void ax_mask_to(float (*x)[16], uint64_t kmask, int c
 __device__ __forceinline__ void ax_mask_half(float* x, uint64_t kmask, int causal, int kt0, int q,
                                              int lane, int t, float val = -__builtin_inff()) {
   const int h4 = 32 * t + ((lane >> 5) << 2);
-  const uint64_t km = kmask >> h4;
   const int lim = causal ? q - kt0 - h4 : AX_BN;
+  uint32_t km = (uint32_t)(kmask >> h4);
+  if (lim < 0) km = 0;
+  else if (lim < 31) km &= (2u << lim) - 1;
 #pragma unroll
-  for (int r = 0; r < 16; ++r) {
-    const int c = ((r >> 2) << 3) + (r & 3);
-    const bool ok = ((km >> c) & 1ull) && c <= lim;
-    x[r] = ok ? x[r] : val;
-  }
+  for (int r = 0; r < 16; ++r) x[r] = ((km >> (((r >> 2) << 3) + (r & 3))) & 1u) ? x[r] : val;
 }
 
 // ---- wave softmax (S <= 2048): expf and the division, bit for bit --------
@@ -540,14 +588,6 @@ __device__ __forceinline__ bool ax_wave_exps(float (*x)[16], bool need_mask, uin
       for (int r = 0; r < 16; ++r) x[t][r] = expf(x[t][r]);
   }
   return fast;
-}
-
-// x = s - m, where for an exact (power-of-two) scale s = round(acc) * scale
-// is formed inside one fma (the product is exact, so this equals the eager
-// subtraction).
-template <bool EXACT_SCALE>
-__device__ __forceinline__ float ax_shift(float v, float scale, float m) {
-  return EXACT_SCALE ? __builtin_fmaf(v, scale, -m) : v - m;
 }
 
 // Key-validity bits of a tile (bit k: key kt0 + k exists and is valid).
@@ -772,17 +812,7 @@ __global__ __launch_bounds__(AX_THREADS, 3) void attn_stats2_kernel(AttnArgs a) 
     ring_barrier<63>();  // pa_max visible; pass B's K loads stay in flight
     mx = fmaxf(mx, pa_max[wave ^ 1][lane & 31]);
     dead = (mx == NEG_INF);
-    if (!dead) {
-      float hi = mx, unused = 0.f;
-      ax_round2<T>(hi, unused);
-      if (!EXACT_SCALE) {
-        hi *= a.scale;
-        ax_round2<T>(hi, unused);
-        m = hi;
-      } else {
-        m = hi * a.scale;
-      }
-    }
+    if (!dead) m = ax_row_max<T, EXACT_SCALE>(mx, a.scale);
   }
 
   // ---- pass B (steps n_live .. 2 n_live-1): e = exp(s - m) into the ATen slots.
@@ -798,12 +828,13 @@ __global__ __launch_bounds__(AX_THREADS, 3) void attn_stats2_kernel(AttnArgs a) 
     const uint64_t kmask = ax_key_mask(kv, kt0, S, lane);
     const bool need_mask = __builtin_amdgcn_readfirstlane(
         (int)((a.causal && (kt0 + AX_BN - 1 > q0w)) || (kmask != ~0ull))) != 0;
-    ax_round_scores<T, EXACT_SCALE>(s, a.scale);
+    AxScores<T, EXACT_SCALE> sc;
+    sc.round(s, a.scale);
     float ev[2][16];
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
-      for (int r = 0; r < 16; ++r) ev[t][r] = ax_shift<EXACT_SCALE>(s[t][r], a.scale, m);
+      for (int r = 0; r < 16; ++r) ev[t][r] = sc.shift(t, r, a.scale, m);
     if (SMK == 1) {
       if (need_mask) ax_mask(ev, kmask, a.causal, kt0, myq, lane);
 #pragma unroll
@@ -978,11 +1009,11 @@ __global__ __launch_bounds__(AX_THREADS, HD == 64 && !SINGLE ? 3 : 2) void attn_
     // Wave-uniform, so that unmasked tiles take a scalar branch around the masking.
     const bool need_mask = __builtin_amdgcn_readfirstlane(
         (int)((a.causal && (kt0 + AX_BN - 1 > q0w)) || (kmask != ~0ull))) != 0;
-    ax_round_scores<T, EXACT_SCALE>(s, a.scale);
+    AxScores<T, EXACT_SCALE> sc;
+    sc.round(s, a.scale);
     float x[2][16];       // this tile's exponentials (wave softmax) or shifted scores
     bool fast_e = false;  // the wave softmax's exps took the in-range sequence
     if constexpr (SINGLE) {
-      // max of the rounded scores = the rounding of the raw max (monotone).
       float mv[2][16];
 #pragma unroll
       for (int t = 0; t < 2; ++t)
@@ -996,12 +1027,12 @@ __global__ __launch_bounds__(AX_THREADS, HD == 64 && !SINGLE ? 3 : 2) void attn_
         for (int r = 0; r < 16; ++r) mx = fmaxf(mx, mv[t][r]);
       mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
       const bool dead = (mx == NEG_INF);
-      m = dead ? 0.f : (EXACT_SCALE ? mx * a.scale : mx);
+      m = dead ? 0.f : ax_row_max<T, EXACT_SCALE>(mx, a.scale);
       float part[32];
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) mv[t][r] = ax_shift<EXACT_SCALE>(s[t][r], a.scale, m);
+        for (int r = 0; r < 16; ++r) mv[t][r] = sc.shift(t, r, a.scale, m);
       fast_e = ax_wave_exps(mv, need_mask, kmask, a.causal, kt0, myq, lane);
 #pragma unroll
       for (int t = 0; t < 2; ++t)
@@ -1019,7 +1050,7 @@ __global__ __launch_bounds__(AX_THREADS, HD == 64 && !SINGLE ? 3 : 2) void attn_
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) x[t][r] = ax_shift<EXACT_SCALE>(s[t][r], a.scale, m);
+        for (int r = 0; r < 16; ++r) x[t][r] = sc.shift(t, r, a.scale, m);
       if (SMK == 1) {
         if (need_mask) ax_mask<PERM>(x, kmask, a.causal, kt0, myq, lane);
       } else {
@@ -1171,7 +1202,9 @@ __global__ __launch_bounds__(AX_THREADS, 2) void attn_rowres_kernel(AttnArgs a) 
       for (int ks = 0; ks < HD / 16; ++ks) kf[t][ks] = __builtin_bit_cast(vec, ld128(krow + 16 * ks));
     }
   };
-  f32x16 s[TMAX][2];
+  AxScores<T, EXACT_SCALE> sc[TMAX];
+  float ev[TMAX][2][16];  // exponentials, then p
+  float mx = NEG_INF;     // of the raw accumulators
   uint64_t kmask[TMAX];
   bool need_mask[TMAX];
   vec kf[2][2][HD / 16];  // two tiles' fragments: the current and the next
@@ -1184,63 +1217,53 @@ __global__ __launch_bounds__(AX_THREADS, 2) void attn_rowres_kernel(AttnArgs a) 
       const int kt0 = (kt_begin + j) * AX_BN;
       if (j + 1 < n_mine) kload(kt0 + AX_BN, kf[(j + 1) & 1]);
       __builtin_amdgcn_sched_barrier(0);
+      f32x16 s[2];
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) s[j][t][r] = 0.f;
+        for (int r = 0; r < 16; ++r) s[t][r] = 0.f;
 #pragma unroll
       for (int ks = 0; ks < HD / 16; ++ks)
 #pragma unroll
-        for (int t = 0; t < 2; ++t) s[j][t] = Mfma<T>::mma32(kf[j & 1][t][ks], qf[ks], s[j][t]);
-      ax_round_scores<T, EXACT_SCALE>(s[j], a.scale);
+        for (int t = 0; t < 2; ++t) s[t] = Mfma<T>::mma32(kf[j & 1][t][ks], qf[ks], s[t]);
+      sc[j].round(s, a.scale);
       kmask[j] = ax_key_mask(kv, kt0, S, lane);
       need_mask[j] = __builtin_amdgcn_readfirstlane(
                          (int)((a.causal && (kt0 + AX_BN - 1 > q0)) || (kmask[j] != ~0ull))) != 0;
-    }
-    __builtin_amdgcn_sched_barrier(0);
-  }
-
-  // ---- row max over the four runs
-  float mx = NEG_INF;
-#pragma unroll
-  for (int j = 0; j < TMAX; ++j) {
-    if (j < n_mine) {
       float mv[2][16];
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) mv[t][r] = s[j][t][r];
-      if (need_mask[j]) ax_mask(mv, kmask[j], a.causal, (kt_begin + j) * AX_BN, myq, lane);
+        for (int r = 0; r < 16; ++r) mv[t][r] = s[t][r];
+      if (need_mask[j]) ax_mask(mv, kmask[j], a.causal, kt0, myq, lane);
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int r = 0; r < 16; ++r) mx = fmaxf(mx, mv[t][r]);
     }
+    __builtin_amdgcn_sched_barrier(0);
   }
+
+  // ---- row max over the four runs
   mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
   if (half == 0) red_max[wave][col] = mx;
   __syncthreads();
   mx = fmaxf(fmaxf(red_max[0][col], red_max[1][col]), fmaxf(red_max[2][col], red_max[3][col]));
   // A row with no admissible key: m = 0, every exponential is 0, l = 1 below.
   const bool dead = (mx == NEG_INF);
-  const float m = dead ? 0.f : (EXACT_SCALE ? mx * a.scale : mx);
+  const float m = dead ? 0.f : ax_row_max<T, EXACT_SCALE>(mx, a.scale);
 
-  // ---- e = expf(s - m), in place
+  // ---- e = expf(s - m)
   bool fast[TMAX];
 #pragma unroll
   for (int j = 0; j < TMAX; ++j) {
     fast[j] = true;
     if (j < n_mine) {
-      float x[2][16];
 #pragma unroll
       for (int t = 0; t < 2; ++t)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) x[t][r] = ax_shift<EXACT_SCALE>(s[j][t][r], a.scale, m);
-      fast[j] = ax_wave_exps(x, need_mask[j], kmask[j], a.causal, (kt_begin + j) * AX_BN, myq, lane);
-#pragma unroll
-      for (int t = 0; t < 2; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) s[j][t][r] = x[t][r];
+        for (int r = 0; r < 16; ++r) ev[j][t][r] = sc[j].shift(t, r, a.scale, m);
+      fast[j] = ax_wave_exps(ev[j], need_mask[j], kmask[j], a.causal, (kt_begin + j) * AX_BN, myq, lane);
     }
   }
 
@@ -1260,7 +1283,7 @@ __global__ __launch_bounds__(AX_THREADS, 2) void attn_rowres_kernel(AttnArgs a) 
 #pragma unroll
           for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) part[16 * t + r] += s[j][t][r];
+            for (int r = 0; r < 16; ++r) part[16 * t + r] += ev[j][t][r];
         }
 #pragma unroll
       for (int i = 0; i < 32; ++i) chain[i][lane] = part[i];
@@ -1310,12 +1333,12 @@ __global__ __launch_bounds__(AX_THREADS, 2) void attn_rowres_kernel(AttnArgs a) 
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) s[j][t][r] = ax_div_fast(s[j][t][r], l, rr);
+          for (int r = 0; r < 16; ++r) ev[j][t][r] = ax_div_fast(ev[j][t][r], l, rr);
       } else {
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) s[j][t][r] = s[j][t][r] / l;
+          for (int r = 0; r < 16; ++r) ev[j][t][r] = ev[j][t][r] / l;
       }
       // Slot (t, r) holds key kt0 + 32 t + 8 (r >> 2) + 4 half + (r & 3):
       // four consecutive keys per r >> 2, one 8-byte write.
@@ -1324,8 +1347,8 @@ __global__ __launch_bounds__(AX_THREADS, 2) void attn_rowres_kernel(AttnArgs a) 
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int rq = 0; rq < 4; ++rq) {
-          const u32x2 pk = u32x2{pack2<T>(s[j][t][4 * rq + 0], s[j][t][4 * rq + 1]),
-                                 pack2<T>(s[j][t][4 * rq + 2], s[j][t][4 * rq + 3])};
+          const u32x2 pk = u32x2{pack2<T>(ev[j][t][4 * rq + 0], ev[j][t][4 * rq + 1]),
+                                 pack2<T>(ev[j][t][4 * rq + 2], ev[j][t][4 * rq + 3])};
           st64(&p_lds[col][kt0 + 32 * t + 8 * rq + 4 * half], pk);
         }
     }
@@ -1425,25 +1448,15 @@ __global__ __launch_bounds__(256) void attn_tile4_kernel(AttnArgs a) {
     }
   }
 
-  // x[4 kb + e] = score of key 32 th + 16 kb + 4 g + e, rounded as eager rounds it.
-  float x[8];
+  // acc8[4 kb + e] = raw score of key 32 th + 16 kb + 4 g + e.
+  float acc8[8];
 #pragma unroll
   for (int kb = 0; kb < 2; ++kb) {
     f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int kc = 0; kc < 2; ++kc) acc = Mfma16<T>::mma(kf[kb][kc], qf[kc], acc);
 #pragma unroll
-    for (int e = 0; e < 4; e += 2) {
-      float u = acc[e], v = acc[e + 1];
-      ax_round2<T, false>(u, v);
-      if (!EXACT_SCALE) {
-        u *= a.scale;
-        v *= a.scale;
-        ax_round2<T>(u, v);
-      }
-      x[4 * kb + e] = u;
-      x[4 * kb + e + 1] = v;
-    }
+    for (int e = 0; e < 4; ++e) acc8[4 * kb + e] = acc[e];
   }
   const uint64_t kmask = ax_key_mask(hp.kv, 0, S, lane);
   const bool need_mask = __builtin_amdgcn_readfirstlane(
@@ -1463,7 +1476,7 @@ __global__ __launch_bounds__(256) void attn_tile4_kernel(AttnArgs a) {
   {
     float mv[8];
 #pragma unroll
-    for (int i = 0; i < 8; ++i) mv[i] = x[i];
+    for (int i = 0; i < 8; ++i) mv[i] = acc8[i];
     if (need_mask) mask8(mv, NEG_INF);
 #pragma unroll
     for (int i = 0; i < 8; ++i) mx = fmaxf(mx, mv[i]);
@@ -1474,11 +1487,19 @@ __global__ __launch_bounds__(256) void attn_tile4_kernel(AttnArgs a) {
   ring_barrier<63>();  // LDS only: nothing of this wave's memory reads waits here
   mx = fmaxf(mx, red_max[th ^ 1][16 * qh + c16]);
   const bool dead = (mx == NEG_INF);
-  const float m = dead ? 0.f : (EXACT_SCALE ? mx * a.scale : mx);
+  const float m = dead ? 0.f : ax_row_max<T, EXACT_SCALE>(mx, a.scale);
 
   // e = expf(s - m), 0 on masked keys.
+  float x[8];
+  {
+    f32x16 av = {};
 #pragma unroll
-  for (int i = 0; i < 8; ++i) x[i] = ax_shift<EXACT_SCALE>(x[i], a.scale, m);
+    for (int i = 0; i < 8; ++i) av[i] = acc8[i];
+    AxScores<T, EXACT_SCALE, 1> sc;
+    sc.round(&av, a.scale);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) x[i] = sc.shift(0, i, a.scale, m);
+  }
   float mn = x[0];
 #pragma unroll
   for (int i = 1; i < 8; ++i) mn = fminf(mn, x[i]);
@@ -1938,12 +1959,12 @@ static int launch_exact_typed(const AttnArgs& a0, hipStream_t st) {
   const long total = (long)nq * a.batch * a.heads;
   if (total > 0x7fffffffL) return TX_EUNSUPPORTED;
   dim3 grid((unsigned)total);
-  // A power-of-two scale makes round(round(acc) * scale) = round(acc) *
-  // scale exactly -- in bf16 always (fp32's exponent range), in fp16 only
-  // while the product stays normal: below 2^-14 eager's fp16 multiply rounds
-  // it to a subnormal and drops bits.  So only bf16 takes the fused form.
+  // EXACT scores (AxScores): in bf16 a power-of-two scale, whose product with
+  // a bf16 value is exact (fp32's exponent range); in fp16 a scale that is an
+  // fp16 value, so that the packed multiply rounds once, as eager does.
   int e2 = 0;
-  const bool exact = std::is_same<T, bf16>::value && (frexpf(a.scale, &e2) == 0.5f);
+  const bool exact = std::is_same<T, bf16>::value ? frexpf(a.scale, &e2) == 0.5f
+                                                  : (float)(_Float16)a.scale == a.scale;
   if (a.head_dim == 64)
     return exact ? launch_layout<T, 64, true>(a, grid, st) : launch_layout<T, 64, false>(a, grid, st);
   if (a.head_dim == 128)
