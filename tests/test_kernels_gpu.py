@@ -883,6 +883,44 @@ def test_online_softmax_key_groups(cuda, dtype, hd, b, h, s, causal, masked, fla
                 assert not o[-1].any()
 
 
+@pytest.fixture
+def rowres():
+    import os
+    old = os.environ.get("TX_ATTN_ROWRES")
+    yield lambda n: os.environ.__setitem__("TX_ATTN_ROWRES", str(n))
+    if old is None:
+        os.environ.pop("TX_ATTN_ROWRES", None)
+    else:
+        os.environ["TX_ATTN_ROWRES"] = old
+
+
+@pytest.mark.parametrize("dtype,hd", [(torch.bfloat16, 64), (torch.float16, 64), (torch.float16, 128),
+                                      (torch.bfloat16, 128)])
+@pytest.mark.parametrize("s,causal,masked", [(1, False, False), (64, True, False), (65, False, True), (129, True, True),
+                                             (256, False, False), (257, True, False), (500, False, True),
+                                             (513, True, True), (1000, False, True), (1024, True, False)])
+def test_exact_attention_row_resident_equals_two_kernels(cuda, dtype, hd, s, causal, masked, rowres):
+    """The row-resident kernel at the edges of its tile runs (one, two and four
+    tiles a wave, waves without a tile) and the two-kernel path: same bits, in
+    both V layouts."""
+    b, h = 2, 3
+    log(f"row-resident s{s} hd{hd} causal={causal} masked={masked} {dtype}")
+    qkv = _randn((b, s, 3 * h * hd), dtype, cuda, 173, 0.8)
+    q, k, v = (qkv[..., j * h * hd:(j + 1) * h * hd].view(b, s, h, hd).transpose(1, 2) for j in range(3))
+    qk = qkv[..., :2 * h * hd].reshape(b * s, 2 * h * hd).contiguous()
+    # The padding columns of V^T hold NaN: nothing may read them into a sum.
+    vt = torch.full((b, h, hd, _C.vt_ld(s)), float("nan"), dtype=dtype, device=cuda)
+    vt[..., :s] = v.transpose(2, 3)
+    valid = (torch.rand((b, s), generator=_gen(174)) < 0.6).to(cuda) if masked else None
+    got = []
+    for n in (0, 1):
+        rowres(n)
+        got.append(_C.flash_attn(qk, vt, b, s, h, hd, hd ** -0.5, causal, key_valid=valid).view(b, s, h, hd).transpose(1, 2))
+        got.append(_C.flash_attn_strided(q, k, v, hd ** -0.5, causal, key_valid=valid))
+    for g in got:
+        assert torch.isfinite(g).all() and torch.equal(g, got[0])
+
+
 @pytest.mark.parametrize("s,hd,causal", [(96, 64, False), (40, 64, False), (17, 64, True), (1500, 64, True),
                                           (2048, 128, False), (1100, 128, True)])
 def test_fully_masked_rows_are_zero_not_nan(cuda, s, hd, causal):

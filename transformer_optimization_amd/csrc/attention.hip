@@ -1128,39 +1128,40 @@ __global__ __launch_bounds__(AX_THREADS, HD == 64 && !SINGLE ? 3 : 2) void attn_
 }
 
 // ============================================================ row-resident
-// attn_rowres_kernel: the eager-exact path for rows of 65 .. 1024 keys at
-// head dim 64 with V head-transposed (the wave softmax), taken for causal
-// rows and for grids the two-kernel path would leave under-filled.  One
+// attn_rowres_kernel: the eager-exact path for rows of up to 1024 keys (the
+// wave softmax), taken for short rows and for grids the two-kernel path would
+// leave under-filled (the rule and its figures: launch_exact_hd).  One
 // workgroup per 32 query rows of one (batch, head); its four waves split
 // the row's live key tiles into four consecutive runs of ceil(tiles / 4).
 // Each wave forms the scores of its run once, from K fragments read
-// straight from global memory, and keeps them in registers (at most 4
-// tiles: 128 values a lane), as ATen's wave softmax holds its row in
-// registers:
+// straight from global memory, and keeps them in registers (at most TMAX
+// tiles, 32 values a lane each), as ATen's wave softmax holds its row in
+// registers.  TMAX = 1, 2, 4 (256, 512, 1024 keys) sizes the registers and the
+// p panel: at 64 x 8 heads x 128 keys TMAX = 1 takes 18.1 us, TMAX = 4 26.1.
 //   * row max: per-wave maxima exchanged through LDS (max is exact and
 //     order-free);
 //   * e = expf(s - m) once per score (the two-kernel path forms it twice);
 //   * row sum in ATen's order: lane slot t of the wave softmax sums the keys
 //     t + 64 it in order of it, and tile it lies in the run of wave it / run,
 //     so the 32 per-lane partial sums pass from wave to wave through LDS
-//     (wave 0 starts from zero, each wave adds its tiles in order), then the
-//     xor butterfly of ax_wave_softmax_sum;
+//     (wave 0 starts from zero, each wave with tiles adds its own in order),
+//     then the xor butterfly of ax_wave_softmax_sum;
 //   * p = e / l, rounded to T into an LDS panel of the 32 rows, and P V on
-//     v_mfma_f32_16x16x32 with each wave running every key in order for 16
-//     head-dim columns: 32 keys per step give the same bits as the
+//     v_mfma_f32_16x16x32 with each wave running every key in order for a
+//     quarter of the head-dim columns: 32 keys per step give the same bits as the
 //     two-kernel path's 32x32x16 chain (16 keys per step).
 // QK^T runs once instead of three times.
 constexpr int AXR_BQ = 32;  // query rows per workgroup
 
-template <typename T, bool EXACT_SCALE>
+template <typename T, int HD, bool EXACT_SCALE, int TMAX, bool VNAT>
 __global__ __launch_bounds__(AX_THREADS, 2) void attn_rowres_kernel(AttnArgs a) {
   typedef typename Mfma<T>::vec vec;
-  constexpr int HD = 64;
-  constexpr int TMAX = 4;  // key tiles per wave (S <= 1024)
-  __shared__ float red_max[4][32];
-  __shared__ float chain[32][64];  // slot sums: 32 values per lane, element-major (no bank conflicts)
+  constexpr int NWV = 4;
+  constexpr int SMAX = NWV * TMAX * AX_BN;
+  __shared__ float red_max[NWV][32];
+  __shared__ f32x4 chain[8][64];  // slot sums: 32 values per lane, four at a time (no bank conflicts)
   // p of the 32 rows, keys contiguous; rows padded by 16 bytes (bank spread).
-  __shared__ __attribute__((aligned(16))) T p_lds[AXR_BQ][1024 + 8];
+  __shared__ __attribute__((aligned(16))) T p_lds[AXR_BQ][SMAX + 8];
 
   const int S = a.seq, H = a.heads;
   const int nq = (S + AXR_BQ - 1) / AXR_BQ;
@@ -1185,7 +1186,8 @@ __global__ __launch_bounds__(AX_THREADS, 2) void attn_rowres_kernel(AttnArgs a) 
   // Live tiles of this block (causal: up to its last row) and this wave's run.
   int n_live = (S + AX_BN - 1) / AX_BN;
   if (a.causal) n_live = min(n_live, min(q0 + AXR_BQ - 1, S - 1) / AX_BN + 1);
-  const int run = (n_live + 3) / 4;
+  const int run = (n_live + NWV - 1) / NWV;
+  const int n_act = (n_live + run - 1) / run;  // waves with a tile
   const int kt_begin = wave * run;
   const int n_mine = max(0, min(run, n_live - kt_begin));  // wave-uniform
   const uint8_t* kv = hp.kv;
@@ -1207,15 +1209,17 @@ __global__ __launch_bounds__(AX_THREADS, 2) void attn_rowres_kernel(AttnArgs a) 
   float mx = NEG_INF;     // of the raw accumulators
   uint64_t kmask[TMAX];
   bool need_mask[TMAX];
-  vec kf[2][2][HD / 16];  // two tiles' fragments: the current and the next
-  if (n_mine > 0) kload(kt_begin * AX_BN, kf[0]);
+  constexpr int KB = TMAX == 1 || HD == 128 ? 1 : 2;  // tiles' fragments held: the current and the next
+  vec kf[KB][2][HD / 16];
+  if (KB == 2 && n_mine > 0) kload(kt_begin * AX_BN, kf[0]);
 #pragma unroll
   for (int j = 0; j < TMAX; ++j) {
     kmask[j] = ~0ull;
     need_mask[j] = false;
     if (j < n_mine) {
       const int kt0 = (kt_begin + j) * AX_BN;
-      if (j + 1 < n_mine) kload(kt0 + AX_BN, kf[(j + 1) & 1]);
+      if (KB == 1) kload(kt0, kf[0]);
+      else if (j + 1 < n_mine) kload(kt0 + AX_BN, kf[(j + 1) % KB]);
       __builtin_amdgcn_sched_barrier(0);
       f32x16 s[2];
 #pragma unroll
@@ -1225,7 +1229,7 @@ __global__ __launch_bounds__(AX_THREADS, 2) void attn_rowres_kernel(AttnArgs a) 
 #pragma unroll
       for (int ks = 0; ks < HD / 16; ++ks)
 #pragma unroll
-        for (int t = 0; t < 2; ++t) s[t] = Mfma<T>::mma32(kf[j & 1][t][ks], qf[ks], s[t]);
+        for (int t = 0; t < 2; ++t) s[t] = Mfma<T>::mma32(kf[j % KB][t][ks], qf[ks], s[t]);
       sc[j].round(s, a.scale);
       kmask[j] = ax_key_mask(kv, kt0, S, lane);
       need_mask[j] = __builtin_amdgcn_readfirstlane(
@@ -1248,7 +1252,8 @@ __global__ __launch_bounds__(AX_THREADS, 2) void attn_rowres_kernel(AttnArgs a) 
   mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
   if (half == 0) red_max[wave][col] = mx;
   __syncthreads();
-  mx = fmaxf(fmaxf(red_max[0][col], red_max[1][col]), fmaxf(red_max[2][col], red_max[3][col]));
+#pragma unroll
+  for (int w = 0; w < NWV; ++w) mx = fmaxf(mx, red_max[w][col]);
   // A row with no admissible key: m = 0, every exponential is 0, l = 1 below.
   const bool dead = (mx == NEG_INF);
   const float m = dead ? 0.f : ax_row_max<T, EXACT_SCALE>(mx, a.scale);
@@ -1267,15 +1272,66 @@ __global__ __launch_bounds__(AX_THREADS, 2) void attn_rowres_kernel(AttnArgs a) 
     }
   }
 
+  // The first V chunks of P V go out here, so that they land while the sums
+  // and divisions run (the barriers below wait for LDS only).  Wave w: head-dim
+  // columns w HD/4 .. +HD/4 - 1 in blocks of 16, both 16-query halves.
+  typedef typename Mfma16<T>::vec vec16;
+  constexpr int NDB = HD / 64;
+  const int r16 = lane & 15, g16 = lane >> 4;
+  const int d_w = wave * (HD / 4);
+  const int n_chunks = n_live * (AX_BN / 32);
+  f32x4 o16[NDB][2];
+#pragma unroll
+  for (int db = 0; db < NDB; ++db)
+#pragma unroll
+    for (int qh = 0; qh < 2; ++qh) o16[db][qh] = f32x4{0.f, 0.f, 0.f, 0.f};
+  // V^T layout: lane's 16 bytes are keys 32 c + 8 (l >> 4) .. +7 of V^T row
+  // d_w + 16 db + (l & 15), the MFMA operand.  Natural layout: head-dim
+  // columns 8 (l & 1) .. +7 of key 32 c + l / 2; the operand is read back
+  // transposed through LDS (v_operand).  Keys at or past S are zero, or (natural)
+  // key S - 1 again: finite values that meet p = 0.
+  auto vchunk = [&](int c, int db) -> u32x4 {
+    if constexpr (VNAT) {
+      const int key = min(32 * c + (lane >> 1), S - 1);
+      return ld128(hp.v + (int64_t)key * a.v_ss + d_w + 16 * db + 8 * (lane & 1));
+    } else {
+      const T* vrow = hp.v + (int64_t)(d_w + 16 * db + r16) * a.ldvt;
+      const int k0 = 32 * c + 8 * g16;
+      u32x4 v = u32x4{0u, 0u, 0u, 0u};
+      if (k0 + 8 <= S) {
+        v = ld128(vrow + k0);
+      } else if (k0 < S) {
+        v = ld128(vrow + k0);
+        int nv = S - k0;  // valid keys of the chunk
+        asm volatile("" : "+v"(nv));  // formed here only (not hoisted)
+#pragma unroll
+        for (int e2 = 0; e2 < 4; ++e2) v[e2] &= (2 * e2 + 1 < nv) ? 0xffffffffu : (2 * e2 < nv ? 0x0000ffffu : 0u);
+      }
+      return v;
+    }
+  };
+  constexpr int VPF = HD == 128 ? 4 : 8;  // V chunks in flight
+  u32x4 vq[VPF][NDB];
+#pragma unroll
+  for (int i = 0; i < VPF; ++i)
+    if (i < n_chunks) {
+#pragma unroll
+      for (int db = 0; db < NDB; ++db) vq[i][db] = vchunk(i, db);
+    }
+
   // ---- row sum: the per-slot partial sums pass through the runs in order
   float part[32];
 #pragma unroll
   for (int i = 0; i < 32; ++i) part[i] = 0.f;
-  for (int w = 0; w < 4; ++w) {
+  for (int w = 0; w < n_act; ++w) {
     if (wave == w) {
       if (w > 0) {
 #pragma unroll
-        for (int i = 0; i < 32; ++i) part[i] = chain[i][lane];
+        for (int i = 0; i < 8; ++i) {
+          const f32x4 c4 = chain[i][lane];
+#pragma unroll
+          for (int e = 0; e < 4; ++e) part[4 * i + e] = c4[e];
+        }
       }
 #pragma unroll
       for (int j = 0; j < TMAX; ++j)
@@ -1286,41 +1342,18 @@ __global__ __launch_bounds__(AX_THREADS, 2) void attn_rowres_kernel(AttnArgs a) 
             for (int r = 0; r < 16; ++r) part[16 * t + r] += ev[j][t][r];
         }
 #pragma unroll
-      for (int i = 0; i < 32; ++i) chain[i][lane] = part[i];
+      for (int i = 0; i < 8; ++i) chain[i][lane] = f32x4{part[4 * i], part[4 * i + 1], part[4 * i + 2], part[4 * i + 3]};
     }
-    __syncthreads();
+    ring_barrier<63>();
   }
 #pragma unroll
-  for (int i = 0; i < 32; ++i) part[i] = chain[i][lane];
+  for (int i = 0; i < 8; ++i) {
+    const f32x4 c4 = chain[i][lane];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) part[4 * i + e] = c4[e];
+  }
   const float l = dead ? 1.f : ax_wave_softmax_sum(part);
   const float rr = ax_div_recip(l);
-
-  // The first V^T chunks of P V go out here, so that they land while the
-  // divisions run (the barrier below waits for LDS only).
-  typedef typename Mfma16<T>::vec vec16;
-  const int r16 = lane & 15, g16 = lane >> 4;
-  const T* vrow = hp.v + (int64_t)(16 * wave + r16) * a.ldvt;
-  const int n_chunks = n_live * (AX_BN / 32);
-  f32x4 o16[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-  auto vchunk = [&](int c) -> u32x4 {
-    const int k0 = 32 * c + 8 * g16;
-    u32x4 v = u32x4{0u, 0u, 0u, 0u};
-    if (k0 + 8 <= S) {
-      v = ld128(vrow + k0);
-    } else if (k0 < S) {
-      v = ld128(vrow + k0);
-      int nv = S - k0;  // valid keys of the chunk
-      asm volatile("" : "+v"(nv));  // formed here only (not hoisted)
-#pragma unroll
-      for (int e2 = 0; e2 < 4; ++e2) v[e2] &= (2 * e2 + 1 < nv) ? 0xffffffffu : (2 * e2 < nv ? 0x0000ffffu : 0u);
-    }
-    return v;
-  };
-  constexpr int VPF = 8;  // V chunks in flight
-  u32x4 vq[VPF];
-#pragma unroll
-  for (int i = 0; i < VPF; ++i)
-    if (i < n_chunks) vq[i] = vchunk(i);
 
   // ---- p = e / l, the correctly rounded division (ax_div_fast where the
   // in-range exponential sequence ran, as attn_pv2_kernel does), rounded to
@@ -1354,38 +1387,63 @@ __global__ __launch_bounds__(AX_THREADS, 2) void attn_rowres_kernel(AttnArgs a) 
     }
   ring_barrier<63>();  // p_lds written; the V^T loads stay in flight
 
-  // ---- P V on v_mfma_f32_16x16x32: wave w owns head-dim columns
-  // 16 w .. 16 w + 15 for both 16-query halves, and runs over every key in
-  // order, 32 per MFMA (the accumulation of the two-kernel path's
-  // 32x32x16 chain, 16 keys per step, gives the same bits: the library's
-  // GEMMs on either instruction agree bit for bit with ours).
-  // A operand: V^T row 16 w + (lane & 15), keys 32 c + 8 (lane >> 4) .. +7,
-  // straight from global memory; B operand: p_lds row 16 qh + (lane & 15),
-  // same keys.  Columns past S are padding of the V^T rows (a chunk that
-  // starts below S ends inside ldvt = round_up(S, 8)): zeroed; chunks at or
-  // past S are not read.
+  // ---- P V on v_mfma_f32_16x16x32: every wave runs over all keys in order
+  // for its head-dim columns, 32 keys per MFMA (the accumulation of the
+  // two-kernel path's 32x32x16 chain, 16 keys per step, gives the same bits:
+  // the library's GEMMs on either instruction agree bit for bit with ours).
+  // A operand: V^T rows (vchunk); B operand: p_lds row 16 qh + (lane & 15).
+  // In the V^T layout columns past S are padding (a chunk that starts below S
+  // ends inside ldvt = round_up(S, 8)): zeroed; chunks at or past S are not
+  // read.
+  // Natural V: the chunk's 32 keys x 16 columns go through a 1 KB buffer of
+  // this wave (one wave's LDS accesses are performed in order: no barrier) and
+  // come back as eight consecutive keys of column l & 15: of two
+  // ds_read_b64_tr_b16, lane j of each 16 addresses key 8 (l >> 4) + 4 r + j / 4,
+  // columns 4 (j % 4) .. +3 (AxVNatOff).
+  __shared__ __attribute__((aligned(16))) T v_lds[VNAT ? 4 * NDB : 1][VNAT ? 512 : 8];
+  auto v_operand = [&](u32x4 v, int db) -> vec16 {
+    if constexpr (VNAT) {
+      T* buf = v_lds[wave * NDB + db];
+      asm volatile("" ::: "memory");
+      st128(buf + 8 * lane, v);
+      const uint32_t addr = (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) T*)buf +
+                            2u * (uint32_t)((8 * g16 + (r16 >> 2)) * 16 + 4 * (r16 & 3));
+      u32x2 lo, hi;
+      asm volatile("ds_read_b64_tr_b16 %0, %2\n\tds_read_b64_tr_b16 %1, %2 offset:128\n\ts_waitcnt lgkmcnt(0)"
+                   : "=&v"(lo), "=&v"(hi) : "v"(addr) : "memory");
+      return __builtin_bit_cast(vec16, u32x4{lo[0], lo[1], hi[0], hi[1]});
+    } else {
+      return __builtin_bit_cast(vec16, v);
+    }
+  };
   for (int c0 = 0; c0 < n_chunks; c0 += VPF) {
 #pragma unroll
     for (int i = 0; i < VPF; ++i) {
       const int c = c0 + i;
       if (c < n_chunks) {
-        const vec16 va = __builtin_bit_cast(vec16, vq[i]);
-        if (c + VPF < n_chunks) vq[i] = vchunk(c + VPF);
+        vec16 pb[2];
 #pragma unroll
-        for (int qh = 0; qh < 2; ++qh) {
-          const vec16 pb = __builtin_bit_cast(vec16, ld128(&p_lds[16 * qh + r16][32 * c + 8 * g16]));
-          o16[qh] = Mfma16<T>::mma(va, pb, o16[qh]);
+        for (int qh = 0; qh < 2; ++qh)
+          pb[qh] = __builtin_bit_cast(vec16, ld128(&p_lds[16 * qh + r16][32 * c + 8 * g16]));
+#pragma unroll
+        for (int db = 0; db < NDB; ++db) {
+          const vec16 va = v_operand(vq[i][db], db);
+          if (c + VPF < n_chunks) vq[i][db] = vchunk(c + VPF, db);
+#pragma unroll
+          for (int qh = 0; qh < 2; ++qh) o16[db][qh] = Mfma16<T>::mma(va, pb[qh], o16[db][qh]);
         }
       }
     }
   }
-  // Lane l: query q0 + 16 qh + (l & 15), head-dim columns 16 w + 4 (l >> 4) .. +3.
+  // Lane l: query q0 + 16 qh + (l & 15), head-dim columns d_w + 16 db + 4 (l >> 4) .. +3.
 #pragma unroll
   for (int qh = 0; qh < 2; ++qh) {
     const int q = q0 + 16 * qh + r16;
     if (q < S) {
-      T* orow = hp.o + (int64_t)q * a.o_ss + 16 * wave + 4 * g16;
-      st64(orow, u32x2{pack2<T>(o16[qh][0], o16[qh][1]), pack2<T>(o16[qh][2], o16[qh][3])});
+      T* orow = hp.o + (int64_t)q * a.o_ss + d_w + 4 * g16;
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+        st64(orow + 16 * db, u32x2{pack2<T>(o16[db][qh][0], o16[db][qh][1]), pack2<T>(o16[db][qh][2], o16[db][qh][3])});
     }
   }
 }
@@ -1909,26 +1967,37 @@ static int launch_exact_hd(const AttnArgs& a, dim3 grid, hipStream_t st) {
       }
     }
   } else if (a.seq <= 2048) {
-    // Wave softmax.  Head dim 64, V^T layout, up to 1024 keys: the
-    // row-resident kernel where it is faster
-    // (measured, same bits): causal rows (runs of about half the tiles), and
-    // shapes whose 128-query blocks would leave CUs idle (fewer than two
-    // workgroups per CU; it launches four times as many).  Long full rows on
-    // a full grid keep the two-kernel path: there the row-resident kernel's
-    // four-tile runs (two waves per SIMD, waits at its hand-offs) measured
-    // 13% slower (c3: 192 vs 169 us).  TX_ATTN_ROWRES=0 / =1 forces either
-    // path (A/B timing only).
-    static const int rowres_env = [] {
-      const char* e = getenv("TX_ATTN_ROWRES");
-      return e ? (e[0] == '0' ? 0 : 1) : -1;
-    }();
-    const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
-    const long blocks128 = (long)grid.x;
-    const bool rowres = rowres_env >= 0 ? rowres_env == 1 : (a.causal || blocks128 < 2L * cus);
-    if (HD == 64 && !VNAT && rowres && a.seq <= 1024) {
+    // Wave softmax, up to 1024 keys: the row-resident kernel where it is
+    // faster (same bits).  It forms each score once, but its waves hold the
+    // row in registers and wait for one another at the hand-offs; the
+    // two-kernel path needs a full grid of 128-query blocks, three per CU.
+    // Largest grid of such blocks, in workgroups per CU, that takes it
+    // (us, two-kernel / row-resident):
+    //   head dim 64: up to 256 keys any (128 x 16 x 256 168 / 157, 8 x 16 x 256
+    //   21.0 / 15.0); up to 512 keys four (32 x 8 x 512 causal 60.5 / 57.8, 64 x
+    //   8 x 512 155 / 166, 8 x 8 x 512 35.8 / 26.0); up to 1024 two (4 x 16 x
+    //   1000 90 / 86, 8 x 16 x 1024 156 / 185, 1 x 8 x 1000 59.9 / 18.7).
+    //   head dim 128: up to 256 keys four, causal any (64 x 16 x 256 137 / 156,
+    //   causal 138 / 131); up to 512 one, causal two (8 x 8 x 512 46.4 / 40.0, 16
+    //   x 8 x 512 67.8 / 72.6, causal 51.9 / 50.3); up to 1024 one (2 x 16 x 1000
+    //   79.7 / 68.8), half of one for full rows of natural V (78 / 101).
+    // TX_ATTN_ROWRES=0 / =1 forces either path (tests and timing).
+    const char* e = getenv("TX_ATTN_ROWRES");
+    const long cus = device_cu_count() > 0 ? device_cu_count() : 256;
+    const long any = 0x7fffffffL;
+    long most;  // blocks of 128 queries
+    if (HD == 64) most = a.seq <= 256 ? any : a.seq <= 512 ? 4 * cus : 2 * cus;
+    else if (a.seq <= 256) most = a.causal ? any : 4 * cus;
+    else if (a.seq <= 512) most = a.causal ? 2 * cus : cus;
+    else most = VNAT && !a.causal ? cus / 2 : cus;
+    const bool rowres = e ? e[0] != '0' : (long)grid.x <= most;
+    if (rowres && a.seq <= 1024) {
       const long total = (long)((a.seq + AXR_BQ - 1) / AXR_BQ) * a.batch * a.heads;
       if (total > 0x7fffffffL) return TX_EUNSUPPORTED;
-      attn_rowres_kernel<T, EXACT><<<dim3((unsigned)total), block, 0, st>>>(a);
+      const dim3 rgrid((unsigned)total);
+      if (a.seq <= 256) attn_rowres_kernel<T, HD, EXACT, 1, VNAT><<<rgrid, block, 0, st>>>(a);
+      else if (a.seq <= 512) attn_rowres_kernel<T, HD, EXACT, 2, VNAT><<<rgrid, block, 0, st>>>(a);
+      else attn_rowres_kernel<T, HD, EXACT, 4, VNAT><<<rgrid, block, 0, st>>>(a);
     } else {
       attn_stats2_kernel<T, HD, EXACT, 0><<<grid, block, 0, st>>>(a);
       attn_pv2_kernel<T, HD, EXACT, 0, false, VNAT><<<grid, block, 0, st>>>(a);
