@@ -1212,16 +1212,18 @@ static int hp_width(const GemmArgs& g, int cus) {
   return best;
 }
 
-// Modelled time (us) of gemm_hp_kernel at a tile width: c + rounds (a k + e),
-// fitted to the same 170 random shapes as gemm_ring_kernel's configurations
-// (standard error 12-13%).
-static double hp_model_us(const GemmArgs& g, int cus, int bn) {
+// Modelled time (us) of gemm_hp_kernel at a tile width: c + rounds (a k + e +
+// gelu g), fitted to the same random shapes as gemm_ring_kernel's
+// configurations (standard error 8-9%).
+static double hp_model_us(const GemmArgs& gm, int cus, int bn) {
   const int i = bn == 256 ? 0 : bn == 192 ? 1 : 2;
-  static const double c[3] = {0.0, 0.0, 0.836}, a[3] = {0.0212, 0.0169, 0.0117}, e[3] = {12.1, 10.3, 7.32};
-  const long tiles = (long)((g.m + 255) / 256) * ((g.n + bn - 1) / bn);
+  static const double c[3] = {0.0, 0.0402, 0.666}, a[3] = {0.0224, 0.018, 0.0123}, e[3] = {10.1, 8.55, 6.29},
+                      g[3] = {7.59, 5.17, 3.77};
+  const long tiles = (long)((gm.m + 255) / 256) * ((gm.n + bn - 1) / bn);
   const long rounds = (tiles + cus - 1) / cus;
-  return c[i] + (double)rounds * (a[i] * g.k + e[i]);
+  return c[i] + (double)rounds * (a[i] * gm.k + e[i] + ((gm.epi & TX_EPI_GELU_ERF) ? g[i] : 0.0));
 }
+
 
 template <typename T, typename TC, typename TB, typename TR, bool QKV>
 static int launch_gemm_typed(const GemmArgs& g0, hipStream_t st) {
@@ -1267,7 +1269,7 @@ static int launch_gemm_typed(const GemmArgs& g0, hipStream_t st) {
   };
   double ring_us = 0.0;
   const bool ring_ks4 = skinny_ok && lsu4;
-  const int ring_cfg = ring_pick(g.m, g.n, g.k, cus, ring_ks4, &ring_us);
+  const int ring_cfg = ring_pick(g.m, g.n, g.k, g.epi & TX_EPI_GELU_ERF, cus, ring_ks4, &ring_us);
   if (variant >= 1000 && variant < 1006 && ring_ok) return ring(variant - 1000, ring_ks4 && variant < 1002);
   // Small M: 16 x 16 blocks while they are few (c2's shapes: 64x1536x512 4.9
   // against 5.3 us), ring tiles (same bits) where the blocks' operand reads
@@ -1317,7 +1319,7 @@ static int launch_gemm_typed(const GemmArgs& g0, hipStream_t st) {
     hp_us = hp_model_us(g, cus, variant);
     // gemm_hp_kernel writes V^T element by element when a 16-row chunk can
     // span two sequences; gemm_ring_kernel does not (S = 421, 2105x3072x1024:
-    // 24.3 against 21.2 us, where the model has 20.1 and 20.9).
+    // 24.3 against 21.2 us, where the model has 19.6 and 20.7).
     if (QKV && g.seq % 16 != 0) hp_us *= 1.2;
     if (big128) variant = 20;
     // Smaller tiles where their modelled time is less (ring_pick), and for

@@ -360,39 +360,41 @@ static int launch_cfg(const GemmArgs& g0, hipStream_t st) {
   return hipGetLastError() == hipSuccess ? TX_OK : TX_EHIP;
 }
 
-// Tile configurations: BM, BN, the LDS stages that NS K steps of them take,
-// workgroups resident per CU, and the launch time's model
-//   t = c + rounds (a k + e),
+// Tile configurations: BM, BN, workgroups resident per CU (LDS stages in
+// launch_typed), and the launch time's model
+//   t = c + rounds (a k + e + gelu g),
 // rounds of at most `per_cu` tiles a CU; a last round of at most one tile a
-// CU runs at its own rate (a1, e1).  Least squares over 170 random shapes
-// (M 257 .. 12000, N and K the projections and MLPs of d_model 256 .. 2048,
-// operands rotated through six sets; standard error 7-12%), microseconds.
-// Picking the least modelled time is 2% off the best configuration of each
-// shape, and 1.65 times the speed of the 256-row tiles alone (geometric mean;
-// at M = 1024, N = 512, K = 2048: 28 -> 9.4 us).
+// CU runs at its own rate (a1, e1, g / 2).  Least squares over 290 random
+// shapes (M 257 .. 20000, N and K the projections and MLPs of d_model 256 ..
+// 2048, operands rotated through six sets; standard error 6-10%),
+// microseconds.  Picking the least modelled time is 1-3% off the best
+// configuration of each shape, and against the 256-row tiles alone 1.65 times
+// the speed up to M = 12000 (geometric mean; at M = 1024, N = 512, K = 2048: 28 ->
+// 9.4 us) and 1.07 times over M 2600 .. 20000 at d_model 1024 and 2048.
 struct RingCfg {
   int bm, bn, per_cu;
-  double c, a, e, a1, e1;
+  double c, a, e, g, a1, e1;
 };
 static const RingCfg RING[] = {
-    {64, 64, 2, 2.74, 0.00572, 1.89, 0.0035, 1.11},    // 4 stages, 64 KB
-    {64, 128, 1, 1.67, 0.00481, 2.86, 0.00481, 2.86},  // 4 stages, 96 KB
-    {128, 128, 1, 1.19, 0.00687, 4.79, 0.00687, 4.79}, // 4 stages, 128 KB
-    {128, 128, 2, 1.37, 0.0144, 4.82, 0.0105, 3.5},    // 2 stages, 64 KB
-    {128, 192, 1, 0.0, 0.00864, 7.16, 0.00864, 7.16},  // 3 stages, 120 KB
-    {128, 192, 2, 3.23, 0.0178, 7.46, 0.0119, 2.83},   // 2 stages, 80 KB
+    {64, 64, 2, 2.76, 0.00568, 1.73, 0.613, 0.00356, 0.965},
+    {64, 128, 1, 1.69, 0.00484, 2.54, 1.05, 0.00484, 2.54},
+    {128, 128, 1, 0.967, 0.00727, 4.27, 2.16, 0.00727, 4.27},
+    {128, 128, 2, 2.48, 0.0144, 3.43, 3.47, 0.0108, 1.82},
+    {128, 192, 1, 0.0, 0.00923, 6.13, 3.27, 0.00923, 6.13},
+    {128, 192, 2, 2.43, 0.0185, 5.66, 5.3, 0.0121, 2.94},
 };
 
 // The configuration of least modelled time for the shape (us in *cost); ks4:
 // of those that have the four-sum order.
-int ring_pick(int m, int n, int k, int cus, bool ks4, double* cost) {
+int ring_pick(int m, int n, int k, bool gelu, int cus, bool ks4, double* cost) {
   int best = 0;
   for (int c = 0; c < (ks4 ? 2 : (int)(sizeof(RING) / sizeof(RING[0]))); ++c) {
     const RingCfg& r = RING[c];
     const long tiles = (long)((m + r.bm - 1) / r.bm) * ((n + r.bn - 1) / r.bn), slots = (long)cus * r.per_cu;
     const long full = tiles / slots, rem = tiles - full * slots;
-    double t = r.c + (double)full * (r.a * k + r.e);
-    if (rem > 0) t += rem <= cus ? r.a1 * k + r.e1 : r.a * k + r.e;
+    const double g = gelu ? r.g : 0.0;
+    double t = r.c + (double)full * (r.a * k + r.e + g);
+    if (rem > 0) t += rem <= cus ? r.a1 * k + r.e1 + g / r.per_cu : r.a * k + r.e + g;
     if (c == 0 || t < *cost) {
       best = c;
       *cost = t;
@@ -408,10 +410,10 @@ static int launch_typed(const GemmArgs& g, int cfg, bool ks4, hipStream_t st) {
       return ks4 ? launch_cfg<T, TC, TR, QKV, 64, 64, 4, true>(g, st) : launch_cfg<T, TC, TR, QKV, 64, 64, 4>(g, st);
     case 1:
       return ks4 ? launch_cfg<T, TC, TR, QKV, 64, 128, 4, true>(g, st) : launch_cfg<T, TC, TR, QKV, 64, 128, 4>(g, st);
-    case 2: return launch_cfg<T, TC, TR, QKV, 128, 128, 4>(g, st);
-    case 3: return launch_cfg<T, TC, TR, QKV, 128, 128, 2>(g, st);
-    case 4: return launch_cfg<T, TC, TR, QKV, 128, 192, 3>(g, st);
-    case 5: return launch_cfg<T, TC, TR, QKV, 128, 192, 2>(g, st);
+    case 2: return launch_cfg<T, TC, TR, QKV, 128, 128, 4>(g, st);  // 128 KB of LDS
+    case 3: return launch_cfg<T, TC, TR, QKV, 128, 128, 2>(g, st);  // 64 KB
+    case 4: return launch_cfg<T, TC, TR, QKV, 128, 192, 3>(g, st);  // 120 KB
+    case 5: return launch_cfg<T, TC, TR, QKV, 128, 192, 2>(g, st);  // 80 KB
     default: return TX_EUNSUPPORTED;
   }
 }
