@@ -110,6 +110,55 @@ __global__ __launch_bounds__(512) void gemm_ring_kernel(GemmArgs g) {
     else b[q - FM] = *reinterpret_cast<const vec*>(base + b_row + 16 * (q - FM) * BK);
   };
 
+  // ---- the epilogue's reads (bias, residual, row flags; addresses clamped into
+  // the operands) go out first: they do not depend on the products, and at K =
+  // 512 their latency after the K loop was a tenth of the launch.  The residual
+  // may alias C: each value is read here by the lane that writes it.  (Larger
+  // tiles have no registers to hold the residual and read it after the loop.)
+  const bool staged = sizeof(TC) == 2 && g.stage16;
+  constexpr int CPR = BN / 8, CH = BM * CPR / NT;  // staged: 16-byte chunks per row, per thread
+  static_assert(CH * NT == BM * CPR, "chunks per thread");
+  constexpr bool PRE_S = CH <= 2, PRE_D = FM * FN <= 4;
+  typename Raw4<TB>::type braw[FN];
+#pragma unroll
+  for (int j = 0; j < FN; ++j) {
+    braw[j] = {};
+    if (epi & TX_EPI_BIAS) braw[j] = ld_raw4((const TB*)g.bias + min(n0 + wn * TN + 16 * j + 4 * kh, g.n - 4));
+  }
+  u32x4 rres[CH];               // staged
+  bool rok[CH];
+  typename Raw4<TR>::type rraw[FN][FM];  // direct
+  auto load_staged = [&]() {
+#pragma unroll
+    for (int p = 0; p < CH; ++p) {
+      rres[p] = u32x4{0u, 0u, 0u, 0u};
+      rok[p] = true;
+      if (!QKV && (epi & (TX_EPI_RESIDUAL | TX_EPI_MASK_OUT))) {
+        const int ch = p * NT + tid, m = min(m0 + ch / CPR, g.m - 1), n = min(n0 + 8 * (ch % CPR), g.n - 8);
+        if (epi & TX_EPI_RESIDUAL) rres[p] = ld128((const TC*)g.res + (int64_t)m * g.ldr + n);
+        rok[p] = gemm_row_valid(g, m);
+      }
+    }
+  };
+  auto load_direct = [&](int j) {
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+      rraw[j][i] = {};
+      if (!QKV && (epi & TX_EPI_RESIDUAL))
+        rraw[j][i] = ld_raw4((const TR*)g.res + (int64_t)min(m0 + wm * TM + 16 * i + fr, g.m - 1) * g.ldr +
+                             min(n0 + wn * TN + 16 * j + 4 * kh, g.n - 4));
+    }
+  };
+  if constexpr (sizeof(TC) == 2 && PRE_S) {
+    if (staged) load_staged();
+  }
+  if constexpr (PRE_D) {
+    if (!staged) {
+#pragma unroll
+      for (int j = 0; j < FN; ++j) load_direct(j);
+    }
+  }
+
   // ---- prologue
   const int pre = min(NS, KT);
 #pragma unroll
@@ -192,33 +241,16 @@ __global__ __launch_bounds__(512) void gemm_ring_kernel(GemmArgs g) {
 
   // ---------------------------------------------------------------- epilogue
   // acc[j][i][e]: row m0 + wm*TM + 16i + fr, column n0 + wn*TN + 16j + 4kh + e.
-  typename Raw4<TB>::type braw[FN];
-#pragma unroll
-  for (int j = 0; j < FN; ++j) {
-    braw[j] = {};
-    if (epi & TX_EPI_BIAS) braw[j] = ld_raw4((const TB*)g.bias + min(n0 + wn * TN + 16 * j + 4 * kh, g.n - 4));
-  }
-  if (sizeof(TC) == 2 && g.stage16) {
+  if (staged) {
     if constexpr (sizeof(TC) == 2) {
       // Staged through LDS so that C, the residual and V^T move as 16-byte
       // runs of whole rows.
-      constexpr int CPR = BN / 8, CH = BM * CPR / NT;  // chunks per row, per thread
-      static_assert(CH * NT == BM * CPR, "chunks per thread");
       TC* stg = reinterpret_cast<TC*>(lds);
       TC* __restrict__ C = reinterpret_cast<TC*>(g.c);
       // V columns of this tile start at vc (a multiple of 16: whole 16-column
       // blocks are on one side); q / k columns go first, then V.
       const int vc = QKV ? min(max(g.qk_cols - n0, 0), BN) : BN;
-      // The residual rows go out before the rounding and GELU.
-      u32x4 rres[CH];
-#pragma unroll
-      for (int p = 0; p < CH; ++p) {
-        rres[p] = u32x4{0u, 0u, 0u, 0u};
-        if (!QKV && (epi & TX_EPI_RESIDUAL)) {
-          const int ch = p * NT + tid, m = min(m0 + ch / CPR, g.m - 1), n = min(n0 + 8 * (ch % CPR), g.n - 8);
-          rres[p] = ld128((const TC*)g.res + (int64_t)m * g.ldr + n);
-        }
-      }
+      if constexpr (!PRE_S) load_staged();  // before the rounding and GELU
       __syncthreads();  // every wave has read its last fragments
       if (!QKV || vc > 0) {
 #pragma unroll
@@ -247,9 +279,8 @@ __global__ __launch_bounds__(512) void gemm_ring_kernel(GemmArgs g) {
           if (m < g.m && n < g.n && (!QKV || 8 * c < vc)) {
             u32x4 out = ld128(stg + r * ES + 8 * c);
             if (!QKV && ((epi & (TX_EPI_RESIDUAL | TX_EPI_MASK_OUT)) != 0)) {
-              const bool ok = gemm_row_valid(g, m);
-              const bool drop = (epi & TX_EPI_MASK_DELTA) && !ok;
-              const bool zero = (epi & TX_EPI_MASK_OUT) && !ok;
+              const bool drop = (epi & TX_EPI_MASK_DELTA) && !rok[p];
+              const bool zero = (epi & TX_EPI_MASK_OUT) && !rok[p];
               float w8[8];
 #pragma unroll
               for (int e = 0; e < 8; ++e) {
@@ -322,20 +353,13 @@ __global__ __launch_bounds__(512) void gemm_ring_kernel(GemmArgs g) {
     const int n = n0 + wn * TN + 16 * j + 4 * kh;
     float bv[4];
     unpack4<TB>(braw[j], bv);
-    typename Raw4<TR>::type rraw[FM];
-#pragma unroll
-    for (int i = 0; i < FM; ++i) {
-      rraw[i] = {};
-      if (!QKV && (epi & TX_EPI_RESIDUAL))
-        rraw[i] = ld_raw4((const TR*)g.res + (int64_t)min(m0 + wm * TM + 16 * i + fr, g.m - 1) * g.ldr +
-                          min(n, g.n - 4));
-    }
+    if constexpr (!PRE_D) load_direct(j);
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
       const int m = m0 + wm * TM + 16 * i + fr;
       if (n < g.n && m < g.m) {
         float rv[4], a4[4];
-        unpack4<TR>(rraw[i], rv);
+        unpack4<TR>(rraw[j][i], rv);
 #pragma unroll
         for (int e = 0; e < 4; ++e) a4[e] = acc[j][i][e];
         gemm_finish4<TC, QKV>(g, m, n, a4, bv, rv, QKV || gemm_row_valid(g, m));
