@@ -834,28 +834,16 @@ def test_online_softmax_running_max_rebase(cuda, pattern, dtype, hd):
     assert err <= 4 * 2.0 ** -8 * max(exact.abs().max().item(), 1e-3)
 
 
-@pytest.fixture
-def flash_groups():
-    import os
-    old = os.environ.get("TX_ATTN_FLASH")
-    yield lambda n: os.environ.__setitem__("TX_ATTN_FLASH", str(n))
-    if old is None:
-        os.environ.pop("TX_ATTN_FLASH", None)
-    else:
-        os.environ["TX_ATTN_FLASH"] = old
-
-
 @pytest.mark.parametrize("dtype,hd", [(torch.bfloat16, 64), (torch.float16, 64), (torch.bfloat16, 128)])
 @pytest.mark.parametrize("b,h,s,causal,masked", [(1, 2, 1, False, False), (2, 4, 63, True, False),
                                                  (1, 3, 65, True, True), (2, 2, 128, False, True),
                                                  (2, 8, 333, True, False), (1, 4, 449, False, True)])
-def test_online_softmax_key_groups(cuda, dtype, hd, b, h, s, causal, masked, flash_groups):
-    """One and two key groups per workgroup, both V layouts: rows whose second
-    group has no tile or no admissible key, odd and even tile counts, a fully
+def test_online_softmax_short_rows_and_masks(cuda, dtype, hd, b, h, s, causal, masked):
+    """Both V layouts: one to eight key tiles, full and ragged, and a fully
     masked sequence (its rows are 0).  Against fp32 attention: q is rounded
     once more (scaled into log2 units) and p once, 2^-p relative each, so 2^-p
     times a few row magnitudes bounds the difference."""
-    log(f"online groups b{b} h{h} s{s} hd{hd} causal={causal} masked={masked} {dtype}")
+    log(f"online b{b} h{h} s{s} hd{hd} causal={causal} masked={masked} {dtype}")
     qkv = _randn((b, s, 3 * h * hd), dtype, cuda, 171, 0.8)
     q, k, v = (qkv[..., j * h * hd:(j + 1) * h * hd].view(b, s, h, hd).transpose(1, 2) for j in range(3))
     valid = None
@@ -872,15 +860,37 @@ def test_online_softmax_key_groups(cuda, dtype, hd, b, h, s, causal, masked, fla
     vt = torch.zeros((b, h, hd, _C.vt_ld(s)), dtype=dtype, device=cuda)
     vt[..., :s] = v.transpose(2, 3)
     eps = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
-    for n in (1, 2):
-        flash_groups(n)
-        o1 = _C.flash_attn(qk, vt, b, s, h, hd, hd ** -0.5, causal, key_valid=valid, softmax="online")
-        o2 = _C.flash_attn_strided(q, k, v, hd ** -0.5, causal, key_valid=valid, softmax="online")
-        for o in (o1.view(b, s, h, hd).transpose(1, 2), o2):
-            err = (o.float() - ref).abs().amax()
-            assert float(err) <= 8 * eps * float(v.float().abs().amax()), f"{n} groups: {float(err)}"
-            if masked:
-                assert not o[-1].any()
+    o1 = _C.flash_attn(qk, vt, b, s, h, hd, hd ** -0.5, causal, key_valid=valid, softmax="online")
+    o2 = _C.flash_attn_strided(q, k, v, hd ** -0.5, causal, key_valid=valid, softmax="online")
+    for o in (o1.view(b, s, h, hd).transpose(1, 2), o2):
+        err = (o.float() - ref).abs().amax()
+        assert float(err) <= 8 * eps * float(v.float().abs().amax()), float(err)
+        if masked:
+            assert not o[-1].any()
+
+
+@pytest.mark.parametrize("softmax", ["eager", "online"])
+@pytest.mark.parametrize("dtype,hd,h,s,causal", [(torch.bfloat16, 64, 8, 333, False), (torch.float16, 64, 8, 1000, True),
+                                                 (torch.bfloat16, 128, 4, 449, True), (torch.float16, 128, 8, 200, False),
+                                                 (torch.bfloat16, 64, 8, 64, False)])
+def test_attention_of_a_sequence_does_not_depend_on_the_batch(cuda, softmax, dtype, hd, h, s, causal):
+    """One sequence alone (a grid far below the CUs) and as the last of 40 (a
+    grid that fills them): the same bits, in both V layouts."""
+    b = 40
+    log(f"batch independence {softmax} h{h} s{s} hd{hd} causal={causal} {dtype}")
+    qkv = _randn((b, s, 3 * h * hd), dtype, cuda, 175, 0.8)
+
+    def run(t):
+        n = t.shape[0]
+        q, k, v = (t[..., j * h * hd:(j + 1) * h * hd].view(n, s, h, hd).transpose(1, 2) for j in range(3))
+        vt = torch.zeros((n, h, hd, _C.vt_ld(s)), dtype=dtype, device=cuda)
+        vt[..., :s] = v.transpose(2, 3)
+        qk = t[..., :2 * h * hd].reshape(n * s, 2 * h * hd).contiguous()
+        o = _C.flash_attn(qk, vt, n, s, h, hd, hd ** -0.5, causal, softmax=softmax)
+        return o.view(n, s, h, hd).transpose(1, 2), _C.flash_attn_strided(q, k, v, hd ** -0.5, causal, softmax=softmax)
+
+    for alone, batch in zip(run(qkv[-1:]), run(qkv)):
+        assert torch.equal(alone[0], batch[-1])
 
 
 @pytest.fixture

@@ -595,10 +595,10 @@ __device__ __forceinline__ uint64_t ax_key_mask(const uint8_t* kv, int kt0, int 
   return __ballot((kt0 + lane < S) && (kv == nullptr || kv[kt0 + lane] != 0));
 }
 
-__device__ __forceinline__ int ax_n_tiles(int S, int causal, int q0, int bq = AX_BQ) {
+__device__ __forceinline__ int ax_n_tiles(int S, int causal, int q0) {
   int n = (S + AX_BN - 1) / AX_BN;
   if (causal) {
-    const int last_q = min(q0 + bq - 1, S - 1);
+    const int last_q = min(q0 + AX_BQ - 1, S - 1);
     n = min(n, last_q / AX_BN + 1);
   }
   return n;
@@ -1669,45 +1669,33 @@ __global__ __launch_bounds__(256) void attn_tile4_kernel(AttnArgs a) {
 // with a two-stage ring for four waves per SIMD (+2%), and raising the wave
 // priority (s_setprio 1) around the QK^T MFMAs (-1%, within run-to-run
 // spread) or around every MFMA group (+2%).
-//
-// QG x KG waves: QG blocks of 32 queries, and KG groups of waves that take
-// every KG-th key tile; their sums meet in LDS at the end.  One workgroup
-// alone needs about 1 us per tile of its chain (barrier, QK^T, max,
-// exponentials, PV), so a grid that does not fill the CUs several times, and
-// the longest causal rows, are bound by the chain's length: KG = 2 halves it
-// (the launch rule and its figures are at launch_exact_hd).
-template <typename T, int HD, bool VNAT, int QG = 4, int KG = 1>
-__global__ __launch_bounds__(64 * QG * KG, 2) void attn_flash_kernel(AttnArgs a) {
+template <typename T, int HD, bool VNAT>
+__global__ __launch_bounds__(AX_THREADS, 2) void attn_flash_kernel(AttnArgs a) {
   typedef typename Mfma<T>::vec vec;
   typedef AxK<T, HD> KL;
   typedef AxVTile<T, HD, VNAT> VL;
-  constexpr int NW = QG * KG, NTH = 64 * NW, BQ = 32 * QG;
-  static_assert(NW == 4 || NW == 8, "groups of four waves load the tiles");
-  constexpr int TPW = 4 * KG / NW;  // tiles of a stage that each of them loads
-  constexpr int NST = (HD == 128 || KG > 1) ? 2 : 3;
-  constexpr int LPW = (KL::LD + VL::LD) * TPW;
-  constexpr int TILE = KL::ELEMS + VL::ELEMS;
-  __shared__ __attribute__((aligned(16))) T kv_lds[NST][KG * TILE];
+  constexpr int NST = (HD == 128) ? 2 : 3;
+  constexpr int LPW = KL::LD + VL::LD;
+  __shared__ __attribute__((aligned(16))) T kv_lds[NST][KL::ELEMS + VL::ELEMS];
 
   const int S = a.seq, H = a.heads;
-  const int nq = (S + BQ - 1) / BQ;
+  const int nq = (S + AX_BQ - 1) / AX_BQ;
   int bh, qb;
   ax_work_of(nq, a.causal, bh, qb);
   const int b = bh / H, h = bh - b * H;
-  const int q0 = qb * BQ;
+  const int q0 = qb * AX_BQ;
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int half = lane >> 5;
-  const int qg = wave % QG, kg = wave / QG;  // this wave's query block and key group
-  const int q0w = q0 + qg * 32, myq = q0w + (lane & 31);
+  const int q0w = q0 + wave * 32, myq = q0w + (lane & 31);
   const float NEG_INF = -__builtin_inff();
   const float c = a.scale * 1.4426950408889634f;
   AxHead<T> hp;
   hp.init(a, b, h);
 
   KL kl;
-  kl.init(hp.k, a.k_ss, S, wave & 3, lane);
+  kl.init(hp.k, a.k_ss, S, wave, lane);
   VL vl;
-  vl.init(hp, a, S, wave & 3, lane);
+  vl.init(hp, a, S, wave, lane);
   AxKOff<HD> ko;
   ko.init_perm(lane);
   vec qf[HD / 16];
@@ -1727,8 +1715,7 @@ __global__ __launch_bounds__(64 * QG * KG, 2) void attn_flash_kernel(AttnArgs a)
 #pragma unroll
     for (int ks = 0; ks < HD / 16; ++ks) settle(qf[ks]);
   }
-  const int n_tiles = ax_n_tiles(S, a.causal, q0, BQ);
-  const int n_steps = (n_tiles + KG - 1) / KG;
+  const int n_tiles = ax_n_tiles(S, a.causal, q0);
   const uint8_t* kv = hp.kv;
 
   f32x16 o_acc[HD / 32];
@@ -1759,43 +1746,32 @@ __global__ __launch_bounds__(64 * QG * KG, 2) void attn_flash_kernel(AttnArgs a)
   }
   f32x4 lsum = {0.f, 0.f, 0.f, 0.f};
 
-  auto issue = [&](int step) {
-    T* base = kv_lds[step % NST];
-#pragma unroll
-    for (int j = 0; j < TPW; ++j) {
-      const int t = (wave >> 2) * TPW + j, kk = min(step * KG + t, n_tiles - 1);
-      kl.issue(kk, base + t * TILE);
-      vl.issue(kk, base + t * TILE + KL::ELEMS);
-    }
+  auto issue = [&](int kt) {
+    const int kk = min(kt, n_tiles - 1);
+    T* base = kv_lds[kt % NST];
+    kl.issue(kk, base);
+    vl.issue(kk, base + KL::ELEMS);
   };
 #pragma unroll
   for (int s = 0; s < NST - 1; ++s) issue(s);
 
-  for (int step = 0; step < n_steps; ++step) {
-    const int kt = step * KG + kg, kt0 = kt * AX_BN;
-    ring_barrier<LPW * (NST - 2)>();  // the step's tiles
-    const T* Ks = kv_lds[step % NST] + kg * TILE;
-    T* Vs = kv_lds[step % NST] + kg * TILE + KL::ELEMS;
-    if (VL::ZERO_TAIL && (step * KG + KG) * AX_BN > S) {
+  for (int kt = 0; kt < n_tiles; ++kt) {
+    const int kt0 = kt * AX_BN;
+    ring_barrier<LPW * (NST - 2)>();  // tile kt
+    T* Vs = kv_lds[kt % NST] + KL::ELEMS;
+    if (VL::ZERO_TAIL && kt0 + AX_BN > S) {
       // Keys >= S of the last tile: zero V (p is 0 there, and 0 * garbage
       // could be NaN), then make the zeros visible.
-      for (int t = 0; t < KG; ++t) {
-        const int t0 = (step * KG + t) * AX_BN;
-        T* V = kv_lds[step % NST] + t * TILE + KL::ELEMS;
-        if (t0 < S && t0 + AX_BN > S)
-          for (int idx = tid; idx < HD * AX_BN; idx += NTH) {
-            const int d = idx / AX_BN, key = idx % AX_BN;
-            if (t0 + key >= S) V[d * AX_BN + (((key >> 3) ^ ax_swz8(d)) << 3) + (key & 7)] = (T)0.f;
-          }
+      for (int idx = tid; idx < HD * AX_BN; idx += AX_THREADS) {
+        const int d = idx / AX_BN, key = idx % AX_BN;
+        if (kt0 + key >= S) Vs[d * AX_BN + (((key >> 3) ^ ax_swz8(d)) << 3) + (key & 7)] = (T)0.f;
       }
       __syncthreads();
     }
-    issue(step + NST - 1);
-    // Nothing to add: no such tile, or every key after this wave's queries.
-    if (KG > 1 && (kt >= n_tiles || (a.causal && kt0 > q0w + 31))) continue;
+    issue(kt + NST - 1);
     vl.begin(Vs);
     f32x16 sn[2];
-    ax_scores<T, HD>(Ks, qf, ko, sn, &negm);
+    ax_scores<T, HD>(kv_lds[kt % NST], qf, ko, sn, &negm);
     // A use of -mc after both MFMAs: the second then also reads it in place
     // as its C operand instead of copying it into its accumulator first
     // (eight v_mov_b64 per tile).
@@ -1818,7 +1794,8 @@ __global__ __launch_bounds__(64 * QG * KG, 2) void attn_flash_kernel(AttnArgs a)
       for (int r = 0; r < 16; ++r) mx = fmaxf(mx, x[t][r]);
     {
       // The other half of the row: lanes l and l ^ 32 swap on the vector ALU
-      // (a cross-lane read through LDS is ~100 cycles of every tile's chain).
+      // instead of a cross-lane read through LDS (16 heads of 100000 keys 40.5
+      // -> 39.2 ms).
       const auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(uint32_t, mx),
                                                        __builtin_bit_cast(uint32_t, mx), false, false);
       mx = fmaxf(__builtin_bit_cast(float, (uint32_t)sw[0]), __builtin_bit_cast(float, (uint32_t)sw[1]));
@@ -1871,42 +1848,7 @@ __global__ __launch_bounds__(64 * QG * KG, 2) void attn_flash_kernel(AttnArgs a)
       }
     }
   }
-  float l_tot = lsum[0];
-  if constexpr (KG > 1) {
-    // Key group 0 adds the others' sums, all measured from the largest of
-    // their maxima.  A group without an admissible key (m_run = -inf) has
-    // zero sums, and its factor is 0.
-    constexpr int ROW = HD / 2 + 2;  // floats per lane: o, l, m
-    static_assert((KG - 1) * QG * ROW * 64 * 4 <= (int)sizeof(kv_lds), "sums fit the ring");
-    ring_drain();
-    __syncthreads();  // every wave is done with the ring
-    float* red = reinterpret_cast<float*>(kv_lds);
-    if (kg > 0) {
-      float* my = red + ((kg - 1) * QG + qg) * ROW * 64 + lane;
-#pragma unroll
-      for (int t = 0; t < HD / 32; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) my[(16 * t + r) * 64] = o_acc[t][r];
-      my[(HD / 2) * 64] = l_tot;
-      my[(HD / 2 + 1) * 64] = m_run;
-    }
-    __syncthreads();
-    if (kg > 0) return;
-#pragma unroll
-    for (int w = 1; w < KG; ++w) {
-      const float* their = red + ((w - 1) * QG + qg) * ROW * 64 + lane;
-      const float l_w = their[(HD / 2) * 64], m_w = their[(HD / 2 + 1) * 64];
-      const float m_new = fmaxf(m_run, m_w);
-      const float f0 = (m_run == NEG_INF) ? 0.f : exp2f(m_run - m_new);
-      const float f1 = (m_w == NEG_INF) ? 0.f : exp2f(m_w - m_new);
-      m_run = m_new;
-      l_tot = l_tot * f0 + l_w * f1;
-#pragma unroll
-      for (int t = 0; t < HD / 32; ++t)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) o_acc[t][r] = o_acc[t][r] * f0 + their[(16 * t + r) * 64] * f1;
-    }
-  }
+  const float l_tot = lsum[0];
   const float inv = l_tot > 0.f ? 1.0f / l_tot : 0.f;
   if (myq < S) {
     T* orow = hp.o + (int64_t)myq * a.o_ss;
@@ -1930,28 +1872,7 @@ template <typename T, int HD, bool EXACT, bool VNAT>
 static int launch_exact_hd(const AttnArgs& a, dim3 grid, hipStream_t st) {
   dim3 block(AX_THREADS);
   if (a.softmax_mode == TX_SOFTMAX_ONLINE) {
-    // Two key groups per workgroup where the grid of 128-query blocks is at
-    // most one workgroup per CU, causal up to two (half of a causal grid is
-    // short): there the chain over a row's tiles is the time.  Head dim 64:
-    // 64-query blocks of four waves; head dim 128: 128-query blocks of eight
-    // (its tiles are too large to load once per 64 queries).  Measured in us,
-    // one group against two: head dim 64, 96 workgroups of 1500 keys 23.7 / 16.7,
-    // 256 of 1024 18.4 / 16.8, 384 of 1500 32.4 / 35.5; causal 256 of 1024
-    // 18.5 / 13.1, 512 of 2048 33.5 / 31.5, 768 of 3000 54.7 / 59.1.  Head dim
-    // 128: 256 of 1024 27.1 / 23.9, 384 of 1500 51.3 / 56.8; causal 512 of 2048
-    // 52.2 / 45.7, 768 of 3000 85.5 / 98.6.  TX_ATTN_FLASH=1 / =2 forces the
-    // number of groups (tests and timing).
-    const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
-    const char* e = getenv("TX_ATTN_FLASH");
-    const bool two = e ? atoi(e) == 2 : (long)grid.x <= (a.causal ? 2L : 1L) * cus;
-    if (two) {
-      constexpr int QG = HD == 64 ? 2 : 4;
-      const long total = (long)((a.seq + 32 * QG - 1) / (32 * QG)) * a.batch * a.heads;
-      if (total > 0x7fffffffL) return TX_EUNSUPPORTED;
-      attn_flash_kernel<T, HD, VNAT, QG, 2><<<dim3((unsigned)total), dim3(128 * QG), 0, st>>>(a);
-    } else {
-      attn_flash_kernel<T, HD, VNAT><<<grid, block, 0, st>>>(a);
-    }
+    attn_flash_kernel<T, HD, VNAT><<<grid, block, 0, st>>>(a);
   } else if (HD == 64 && a.seq <= AX_BN) {
     // One key tile: the PV kernel forms the row statistics itself.  At head
     // dim 128 that kernel needs more than 256 registers; those rows take the
