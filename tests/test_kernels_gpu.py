@@ -931,6 +931,40 @@ def test_exact_attention_row_resident_equals_two_kernels(cuda, dtype, hd, s, cau
         assert torch.isfinite(g).all() and torch.equal(g, got[0])
 
 
+@pytest.mark.parametrize("hd,s,causal,masked", [(64, 40, False, False), (64, 64, True, True), (64, 200, False, True),
+                                                (64, 1000, True, False), (64, 1500, False, True),
+                                                (64, 2304, False, True), (128, 40, False, True), (128, 300, True, False),
+                                                (128, 1500, True, True), (128, 2304, True, False)])
+def test_rows_that_overflow_to_minus_inf_are_nan_as_in_eager(cuda, hd, s, causal, masked):
+    """fp16 rows whose admissible scores all lie below -65520 (every third
+    query): they round to -inf, and eager's softmax of such a row is NaN.
+    Through every exact kernel (one tile, row-resident, two kernels with the
+    wave and the block softmax), both V layouts: the same rows are NaN, and
+    the others have eager's bits."""
+    b, h = 2, 2
+    log(f"overflow to -inf s{s} hd{hd} causal={causal} masked={masked}")
+    q = _randn((b, h, s, hd), torch.float16, cuda, 181, 0.02)
+    q[:, :, ::3] = 45.0
+    k = _randn((b, h, s, hd), torch.float16, cuda, 182) - 45.0
+    v = _randn((b, h, s, hd), torch.float16, cuda, 183)
+    valid = None
+    if masked:
+        valid = torch.rand((b, s), generator=_gen(184)).to(cuda) < 0.6
+        valid[:, 0] = True  # no query without an admissible key
+    ref = _eager_attention(q, k, v, hd ** -0.5, causal, valid).float()
+    bad = torch.zeros(s, dtype=torch.bool, device=cuda)
+    bad[::3] = True
+    assert torch.equal(ref.isnan().all(-1), bad.expand(b, h, s))
+    qk = torch.cat([t.transpose(1, 2).reshape(b * s, h * hd) for t in (q, k)], 1)
+    vt = torch.zeros((b, h, hd, _C.vt_ld(s)), dtype=torch.float16, device=cuda)
+    vt[..., :s] = v.transpose(2, 3)
+    o1 = _C.flash_attn(qk, vt, b, s, h, hd, hd ** -0.5, causal, key_valid=valid)
+    o2 = _C.flash_attn_strided(q, k, v, hd ** -0.5, causal, key_valid=valid)
+    for o in (o1.view(b, s, h, hd).transpose(1, 2).float(), o2.float()):
+        assert torch.equal(o.isnan(), ref.isnan())
+        assert torch.equal(o.nan_to_num(0.0), ref.nan_to_num(0.0))
+
+
 @pytest.mark.parametrize("s,hd,causal", [(96, 64, False), (40, 64, False), (17, 64, True), (1500, 64, True),
                                           (2048, 128, False), (1100, 128, True)])
 def test_fully_masked_rows_are_zero_not_nan(cuda, s, hd, causal):

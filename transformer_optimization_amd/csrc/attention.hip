@@ -951,15 +951,17 @@ __global__ __launch_bounds__(AX_THREADS, HD == 64 && !SINGLE ? 3 : 2) void attn_
 #pragma unroll
     for (int ks = 0; ks < HD / 16; ++ks) settle(qf[ks]);
   }
-  // Row constants.  A row with no admissible key (m = -inf) gets m = 0 and
-  // l = 1: its scores are all -inf, so p = 0 and o = 0.
+  // Row constants.  A row with no admissible key (its sum is 0) gets m = 0 and
+  // l = 1: its scores are all -inf, so p = 0 and o = 0.  m alone does not tell
+  // such a row: scores that all round to -inf give m = -inf and l = NaN, and
+  // NaN results, as in the kernels that hold the row in registers.
   float m = 0.f, l = 1.f;
   if (!SINGLE && myq < S) {
     const float* st = a.row_stats + ((int64_t)bh * S + myq) * 2;
     m = st[0];
     l = st[1];
   }
-  if (m == NEG_INF) {
+  if (l == 0.f) {
     m = 0.f;
     l = 1.f;
   }
