@@ -230,6 +230,20 @@ int tx_flash_attn_fwd_noalloc(const void* qk, const void* vt, int64_t ldvt, void
                               int64_t batch, int64_t seq, int64_t heads, int64_t head_dim,
                               float scale, int causal, int softmax_mode, int dt, void* stream);
 
+/* tx_select_kernel: for tests and timing, the kernel that the calling thread's
+ * later calls of `op` take where several give the result; no counterpart in
+ * the reference.  variant < 0 restores the process's choice: the dispatcher's
+ * own, or the value that TX_GEMM_VARIANT / TX_ATTN_ROWRES had in the
+ * environment at the first launch (read once: a launch does not look at the
+ * environment, which another thread may be changing).  Variants of
+ * TX_SELECT_GEMM are named at launch_gemm_typed (csrc/gemm.hip); of
+ * TX_SELECT_ATTN_ROWRES: 0 = the two-kernel path, 1 = the row-resident kernel
+ * (rows of up to 1024 keys).  Returns TX_EINVAL for another op.
+ */
+#define TX_SELECT_GEMM 0
+#define TX_SELECT_ATTN_ROWRES 1
+int tx_select_kernel(int op, int variant);
+
 #ifdef __cplusplus
 }
 #endif

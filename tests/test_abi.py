@@ -109,6 +109,15 @@ def test_layernorm_validation_without_gpu():
     assert ln(FAKE, None, None, FAKE, FAKE, FAKE, None, None, None, 4, 64, 1e-5, 2, 2, 1, 2, 0, None) == _C.TX_EUNSUPPORTED
 
 
+def test_select_kernel_validation_without_gpu():
+    lib = _C.load_library()
+    for op in (_C.SELECT_GEMM, _C.SELECT_ATTN_ROWRES):
+        assert lib.tx_select_kernel(op, 1) == _C.TX_OK
+        assert lib.tx_select_kernel(op, -1) == _C.TX_OK
+    for op in (-1, 2):
+        assert lib.tx_select_kernel(op, 0) == _C.TX_EINVAL
+
+
 def test_status_maps_to_exception():
     with pytest.raises(_C.TxError) as info:
         _C._check("tx_gemm", _C.TX_EUNSUPPORTED)

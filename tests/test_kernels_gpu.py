@@ -222,7 +222,7 @@ def test_qkv_proj_layouts(cuda, dtype, b, s, d, h):
 
 
 # The 256-row kernel's three tile widths against the in-order register-staged
-# kernel (TX_GEMM_VARIANT selects the kernel per call; 0 = gemm_kernel): ragged
+# kernel (tx_select_kernel; 0 = gemm_kernel): ragged
 # M and N, N % 8 == 4 (the direct epilogue), K = 64 (one k step per tile), the
 # in-place residual with row masks, GELU, and packed QKV whose sequence length
 # is not a multiple of 16 (V^T written without staging).
@@ -233,17 +233,8 @@ HP_EDGE_SHAPES = [(520, 196, 192), (777, 584, 128), (300, 256, 64), (1000, 1032,
 
 @pytest.fixture
 def gemm_variant():
-    import os
-    old = os.environ.get("TX_GEMM_VARIANT")
-
-    def set_variant(v):
-        os.environ["TX_GEMM_VARIANT"] = str(v)
-
-    yield set_variant
-    if old is None:
-        os.environ.pop("TX_GEMM_VARIANT", None)
-    else:
-        os.environ["TX_GEMM_VARIANT"] = old
+    yield lambda v: _C.select_kernel(_C.SELECT_GEMM, v)
+    _C.select_kernel(_C.SELECT_GEMM, -1)
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
@@ -294,7 +285,7 @@ def test_qkv_proj_unstaged_v_matches_inorder_kernel(cuda, dtype, gemm_variant):
     assert float((qk.float() - ref[:, : 2 * d]).abs().max()) < 0.05
 
 
-# gemm_ring_kernel's tile configurations (TX_GEMM_VARIANT 1000 ..) against the
+# gemm_ring_kernel's tile configurations (variants 1000 ..) against the
 # in-order kernel, bit for bit: one to five K steps (fewer than the ring's
 # stages, equal, more), one tile and a ragged last tile in M and N, N % 8 == 4
 # (the direct epilogue), fp32 results and hi/lo pairs.
@@ -369,6 +360,38 @@ def test_qkv_proj_ring_configurations(cuda, dtype, b, s, d, h, gemm_variant):
         gemm_variant(v)
         qk, vt = run()
         assert torch.equal(qk, qk0) and torch.equal(vt, vt0), f"variant {v}"
+
+
+def test_gemm_kernel_choice_is_per_thread_and_not_the_environment(cuda, gemm_variant, monkeypatch):
+    """Variant 9 adds K in eight parts, which shows in the bits.  Set in the
+    environment after the first launch it changes nothing (no launch reads the
+    environment, which another thread may be writing), and selected in another
+    thread it changes that thread's calls only."""
+    import threading
+
+    log("gemm kernel choice")
+    a = _randn((64, 1024), torch.bfloat16, cuda, 91)
+    w = _randn((64, 1024), torch.bfloat16, cuda, 92)
+    own = _C.gemm(a, w, out_dtype=torch.float32)
+    gemm_variant(9)
+    split = _C.gemm(a, w, out_dtype=torch.float32)
+    gemm_variant(-1)
+    assert not torch.equal(own, split)
+    monkeypatch.setenv("TX_GEMM_VARIANT", "9")
+    assert torch.equal(_C.gemm(a, w, out_dtype=torch.float32), own)
+    monkeypatch.delenv("TX_GEMM_VARIANT")
+    stream, got = torch.cuda.current_stream(), []
+
+    def other():
+        with torch.cuda.stream(stream):
+            _C.select_kernel(_C.SELECT_GEMM, 9)
+            got.append(_C.gemm(a, w, out_dtype=torch.float32))
+
+    t = threading.Thread(target=other)
+    t.start()
+    t.join()
+    assert torch.equal(got[0], split)
+    assert torch.equal(_C.gemm(a, w, out_dtype=torch.float32), own)
 
 
 def test_gemm_wide_row_stride_takes_64bit_kernel(cuda):
@@ -895,13 +918,8 @@ def test_attention_of_a_sequence_does_not_depend_on_the_batch(cuda, softmax, dty
 
 @pytest.fixture
 def rowres():
-    import os
-    old = os.environ.get("TX_ATTN_ROWRES")
-    yield lambda n: os.environ.__setitem__("TX_ATTN_ROWRES", str(n))
-    if old is None:
-        os.environ.pop("TX_ATTN_ROWRES", None)
-    else:
-        os.environ["TX_ATTN_ROWRES"] = old
+    yield lambda n: _C.select_kernel(_C.SELECT_ATTN_ROWRES, n)
+    _C.select_kernel(_C.SELECT_ATTN_ROWRES, -1)
 
 
 @pytest.mark.parametrize("dtype,hd", [(torch.bfloat16, 64), (torch.float16, 64), (torch.float16, 128),

@@ -29,6 +29,7 @@ TX_F32, TX_F16, TX_BF16 = 0, 1, 2
 LN_HAS_DELTA, LN_MASK_DELTA, LN_MASK_X, LN_MASK_OUT, LN_WRITE_X, LN_SPLIT_Y = 1, 2, 4, 8, 16, 32
 EPI_BIAS, EPI_GELU_ERF, EPI_RESIDUAL, EPI_MASK_DELTA, EPI_MASK_OUT, EPI_SPLIT_OUT = 1, 2, 4, 8, 16, 32
 SOFTMAX_EAGER, SOFTMAX_ONLINE = 0, 1
+SELECT_GEMM, SELECT_ATTN_ROWRES = 0, 1
 SOFTMAX_MODES = {"eager": SOFTMAX_EAGER, "online": SOFTMAX_ONLINE}
 # Longest sequence the eager-exact softmax serves (tx_flash_attn_fwd returns
 # TX_EUNSUPPORTED above it: 1024 key tiles of 64); below it, the lengths
@@ -50,6 +51,7 @@ EXPORTED_SYMBOLS = (
     "tx_flash_attn_fwd",
     "tx_flash_attn_fwd_strided",
     "tx_flash_attn_fwd_noalloc",
+    "tx_select_kernel",
 )
 
 # Rows (batch * heads * seq) the fixed scratch of tx_flash_attn_fwd_noalloc holds.
@@ -80,6 +82,8 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.tx_status_string.argtypes = [_i32]
     lib.tx_device_cu_count.restype = _i32
     lib.tx_device_cu_count.argtypes = []
+    lib.tx_select_kernel.restype = _i32
+    lib.tx_select_kernel.argtypes = [_i32, _i32]
     lib.tx_eager_softmax_supported.restype = _i32
     lib.tx_eager_softmax_supported.argtypes = [_i64, _i64]
     lib.tx_layernorm_residual.restype = _i32
@@ -198,6 +202,12 @@ def _dt(t: torch.Tensor) -> int:
 
 def cu_count() -> int:
     return int(load_library().tx_device_cu_count())
+
+
+def select_kernel(op: int, variant: int) -> None:
+    """Tests and timing: the kernel that this thread's later calls of ``op``
+    (``SELECT_GEMM``, ``SELECT_ATTN_ROWRES``) take; -1 restores the choice."""
+    _check("tx_select_kernel", load_library().tx_select_kernel(int(op), int(variant)))
 
 
 _eager_ok: dict = {}

@@ -1,5 +1,6 @@
 // C-ABI entry points: host-side validation, then one launch on the caller's
 // stream.  Nothing here allocates, frees or synchronises.
+#include <cstdlib>
 #include <mutex>
 
 #include "tx_internal.hpp"
@@ -32,6 +33,18 @@ int64_t device_shared_mem_per_block() {
     cache[dev] = v;
   });
   return cache[dev];
+}
+
+static thread_local int thread_kernel[2] = {-1, -1};  // TX_SELECT_*
+
+int selected_kernel(int op) {
+  if (thread_kernel[op] >= 0) return thread_kernel[op];
+  auto env = [](const char* name) {
+    const char* e = getenv(name);
+    return e ? atoi(e) : -1;
+  };
+  static const int process_kernel[2] = {env("TX_GEMM_VARIANT"), env("TX_ATTN_ROWRES")};
+  return process_kernel[op];
 }
 
 static inline bool aligned16(const void* p) { return ((uintptr_t)p & 15u) == 0; }
@@ -70,6 +83,12 @@ int tx_eager_softmax_supported(int64_t seq, int64_t shared_mem_per_block) {
   if (shared_mem_per_block <= 0) shared_mem_per_block = device_shared_mem_per_block();
   if (shared_mem_per_block <= 0) return -1;
   return eager_softmax_mirrorable(seq, shared_mem_per_block) ? 1 : 0;
+}
+
+int tx_select_kernel(int op, int variant) {
+  if (op != TX_SELECT_GEMM && op != TX_SELECT_ATTN_ROWRES) return TX_EINVAL;
+  thread_kernel[op] = variant < 0 ? -1 : variant;
+  return TX_OK;
 }
 
 int tx_layernorm_residual(const void* x, const void* delta, void* x_out, void* y,

@@ -1904,8 +1904,8 @@ static int launch_exact_hd(const AttnArgs& a, dim3 grid, hipStream_t st) {
     //   causal 138 / 131); up to 512 one, causal two (8 x 8 x 512 46.4 / 40.0, 16
     //   x 8 x 512 67.8 / 72.6, causal 51.9 / 50.3); up to 1024 one (2 x 16 x 1000
     //   79.7 / 68.8), half of one for full rows of natural V (78 / 101).
-    // TX_ATTN_ROWRES=0 / =1 forces either path (tests and timing).
-    const char* e = getenv("TX_ATTN_ROWRES");
+    // tx_select_kernel forces either path (tests and timing).
+    const int forced = selected_kernel(TX_SELECT_ATTN_ROWRES);
     const long cus = device_cu_count() > 0 ? device_cu_count() : 256;
     const long any = 0x7fffffffL;
     long most;  // blocks of 128 queries
@@ -1913,7 +1913,7 @@ static int launch_exact_hd(const AttnArgs& a, dim3 grid, hipStream_t st) {
     else if (a.seq <= 256) most = a.causal ? any : 4 * cus;
     else if (a.seq <= 512) most = a.causal ? 2 * cus : cus;
     else most = VNAT && !a.causal ? cus / 2 : cus;
-    const bool rowres = e ? e[0] != '0' : (long)grid.x <= most;
+    const bool rowres = forced >= 0 ? forced != 0 : (long)grid.x <= most;
     if (rowres && a.seq <= 1024) {
       const long total = (long)((a.seq + AXR_BQ - 1) / AXR_BQ) * a.batch * a.heads;
       if (total > 0x7fffffffL) return TX_EUNSUPPORTED;

@@ -232,7 +232,7 @@ __global__ __launch_bounds__(WM* WN * 64) void gemm_kernel(GemmArgs g) {
 
 // ================================================================ big tiles
 // gemm_big_kernel: 128 x 128 / 256 x 256 tiles, compiler-scheduled; the
-// baseline gemm_hp_kernel is measured against (TX_GEMM_VARIANT 20 / 19).
+// baseline gemm_hp_kernel is measured against (variants 20 / 19).
 //
 // Persistent: the grid holds at most as many workgroups as fit on the CUs
 // at once (LDS-bound: one for the default tiles) and workgroup w
@@ -928,7 +928,7 @@ __global__ __launch_bounds__(512, 1) void gemm_hp_kernel(GemmArgs g) {
 // gemm_lsu_kernel runs).  One wave owns a 32 x 32 output block and streams
 // its operand fragments straight from global memory into registers (a ring
 // PF k-steps deep, no LDS).  KSPLIT = 1: the wave runs the whole K in order
-// (bit-identical to the other kernels).  KSPLIT > 1 (TX_GEMM_VARIANT=9, for
+// (bit-identical to the other kernels).  KSPLIT > 1 (variant 9, for
 // comparison only): the workgroup's KSPLIT waves each run one K/KSPLIT slice
 // and the partial sums are added in slice order through LDS.
 template <typename T, typename TC, typename TB, typename TR, int KSPLIT, bool QKV>
@@ -1248,9 +1248,11 @@ static int launch_gemm_typed(const GemmArgs& g0, hipStream_t st) {
   // 128 x BN/2 (one wave per SIMD: 10-60% slower, waits exposed), 32x32x16
   // MFMAs (5-10% slower), BK = 32 with four stages (half-line L2 requests,
   // slower), fragment reads packed at the start of a group (3-5% slower).
-  // TX_GEMM_VARIANT overrides the choice (tuning only).
-  int variant = -1;
-  if (const char* e = getenv("TX_GEMM_VARIANT")) variant = atoi(e);
+  // tx_select_kernel / TX_GEMM_VARIANT override the choice (tests and timing):
+  // 0 gemm_kernel; 8, 9 gemm_skinny_kernel; 10, 11 gemm_lsu_kernel; 19, 20
+  // gemm_big_kernel; 128 to 256, 1283 gemm_hp_kernel; 1000 + i gemm_ring_kernel's
+  // configuration i.  Where one does not take the shape: gemm_kernel.
+  int variant = selected_kernel(TX_SELECT_GEMM);
   const int cus = device_cu_count() > 0 ? device_cu_count() : 256;
   const long t256 = (long)((g.m + 255) / 256) * ((g.n + 255) / 256);
   // Skinny M: fewer 256-row tiles than CUs and at most 256 rows.  K below

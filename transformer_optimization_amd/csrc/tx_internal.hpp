@@ -82,6 +82,9 @@ int launch_gemm_ring(const GemmArgs& g, int ab_dt, int c_dt, int res_dt, bool qk
                      hipStream_t st);
 int launch_attention(const AttnArgs& a, int dt, hipStream_t st);
 int device_cu_count();
+// The variant of op (TX_SELECT_*) that this thread or the process's environment
+// asks for; -1: the dispatcher's own choice.
+int selected_kernel(int op);
 // Shared memory per block of the current device, as the HIP runtime reports
 // it to every library on the device (0 if it cannot be queried).
 int64_t device_shared_mem_per_block();

@@ -1,6 +1,6 @@
 """A/B timing of kernel variants on one GPU, in one process.
 
-The GEMM dispatcher reads ``TX_GEMM_VARIANT`` on every call ("default" = the
+``tx_select_kernel`` sets the GEMM kernel of this thread ("default" = the
 dispatcher's own choice; 20 / 19 = the 128x128 / 256x256 ``gemm_big_kernel``;
 256 / 192 / 128 = ``gemm_hp_kernel`` at that tile width; 0 = the
 register-staged ``gemm_kernel``), so variants of one shape
@@ -20,7 +20,6 @@ its output bitwise against ``torch.native_layer_norm``.
 from __future__ import annotations
 
 import argparse
-import os
 import statistics
 import sys
 
@@ -81,11 +80,11 @@ def ab_gemm(m: int, n: int, k: int, epi: str, dtype: torch.dtype, variants, roun
         for v in variants:
             # Set while the graph is captured: it records the kernel the
             # dispatcher picked for this variant.
-            os.environ["TX_GEMM_VARIANT"] = str(v)
+            _C.select_kernel(_C.SELECT_GEMM, v)
             try:
                 times[v].append(graph_time_us(fns[v], reps))
             finally:
-                os.environ.pop("TX_GEMM_VARIANT", None)
+                _C.select_kernel(_C.SELECT_GEMM, -1)
     flops = 2.0 * m * n * k
     for v in variants:
         same = torch.equal(outs[v], ref)
@@ -123,7 +122,7 @@ def main(argv=None) -> int:
     pg.add_argument("k", type=int)
     pg.add_argument("--epi", choices=("bias", "gelu", "residual"), default="bias")
     pg.add_argument("--variants", default="default,20",
-                    help="comma list of TX_GEMM_VARIANT values; 'default' = the dispatcher's choice")
+                    help="comma list of GEMM variants; 'default' = the dispatcher's choice")
     pl = sub.add_parser("layernorm")
     pl.add_argument("m", type=int)
     pl.add_argument("d", type=int)
