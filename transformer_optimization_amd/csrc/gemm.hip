@@ -25,6 +25,7 @@
 
 #include "common.hpp"
 #include "gemm_common.hpp"
+#include "gemm_route.hpp"
 #include "tx_internal.hpp"
 
 namespace tx {
@@ -1185,46 +1186,6 @@ static int launch_hp(const GemmArgs& g0, hipStream_t st) {
   return hipGetLastError() == hipSuccess ? TX_OK : TX_EHIP;
 }
 
-// Tile width of gemm_hp_kernel for a shape: the least of
-//   w(BN) * BN * (rounds(BN) * K + 1000),
-// rounds = ceil(tiles / CUs) (one workgroup per CU), 1000 ~ the exposed last
-// epilogue and pipeline fill in units of K, w = 0.97, 1, 1.2 for 256, 192,
-// 128 (per-FLOP cost of the narrower wave tiles).  Fitted to every c3/c4
-// GEMM shape with all three widths timed in one process and checked on
-// whole forwards: it picks 256 for c3's FFN-in and c4's out_proj, FFN-in and
-// FFN-out, 192 for the QKV projections, 128 for c3's out_proj and FFN-out.
-// (At c4's QKV the 256-wide tiles win in isolation, 172 vs 181 us, but not
-// inside the forward, where their two K stages see cold operands.)
-static int hp_width(const GemmArgs& g, int cus) {
-  static const int bn[3] = {256, 192, 128};
-  static const double w[3] = {0.97, 1.0, 1.2};
-  int best = 256;
-  double best_cost = 0.0;
-  for (int c = 0; c < 3; ++c) {
-    const long tiles = (long)((g.m + 255) / 256) * ((g.n + bn[c] - 1) / bn[c]);
-    const long rounds = (tiles + cus - 1) / cus;
-    const double cost = w[c] * bn[c] * ((double)rounds * g.k + 1000.0);
-    if (c == 0 || cost < best_cost) {
-      best = bn[c];
-      best_cost = cost;
-    }
-  }
-  return best;
-}
-
-// Modelled time (us) of gemm_hp_kernel at a tile width: c + rounds (a k + e +
-// gelu g), fitted to the same random shapes as gemm_ring_kernel's
-// configurations (standard error 8-9%).
-static double hp_model_us(const GemmArgs& gm, int cus, int bn) {
-  const int i = bn == 256 ? 0 : bn == 192 ? 1 : 2;
-  static const double c[3] = {0.0, 0.0402, 0.666}, a[3] = {0.0224, 0.018, 0.0123}, e[3] = {10.1, 8.55, 6.29},
-                      g[3] = {7.59, 5.17, 3.77};
-  const long tiles = (long)((gm.m + 255) / 256) * ((gm.n + bn - 1) / bn);
-  const long rounds = (tiles + cus - 1) / cus;
-  return c[i] + (double)rounds * (a[i] * gm.k + e[i] + ((gm.epi & TX_EPI_GELU_ERF) ? g[i] : 0.0));
-}
-
-
 template <typename T, typename TC, typename TB, typename TR, bool QKV>
 static int launch_gemm_typed(const GemmArgs& g0, hipStream_t st) {
   GemmArgs g = g0;
@@ -1241,7 +1202,7 @@ static int launch_gemm_typed(const GemmArgs& g0, hipStream_t st) {
                       (!(g.epi & TX_EPI_BIAS) || al(g.bias, 4 * sizeof(TB))) &&
                       (!(g.epi & TX_EPI_RESIDUAL) || ((g.ldr % 4 == 0) && al(g.res, 4 * sizeof(TR))));
   // Tile shape: gemm_hp_kernel (256 x BN, eight waves, hand-ordered
-  // pipeline) with BN from hp_width.  A/B in one process against
+  // pipeline) with BN from gemm_hp_width.  A/B in one process against
   // gemm_big_kernel's 128x128 tiles (2x2 waves of 64x64, two workgroups per
   // CU) and 256x256 tiles (2x4 waves of 128x64): 8-23% faster at every c3/c4
   // shape.  Measured and not chosen (hp kernel): four waves of 128x128 /
@@ -1271,7 +1232,7 @@ static int launch_gemm_typed(const GemmArgs& g0, hipStream_t st) {
   };
   double ring_us = 0.0;
   const bool ring_ks4 = skinny_ok && lsu4;
-  const int ring_cfg = ring_pick(g.m, g.n, g.k, g.epi & TX_EPI_GELU_ERF, cus, ring_ks4, &ring_us);
+  const int ring_cfg = gemm_ring_pick(g.m, g.n, g.k, g.epi & TX_EPI_GELU_ERF, cus, ring_ks4, &ring_us);
   if (variant >= 1000 && variant < 1006 && ring_ok) return ring(variant - 1000, ring_ks4 && variant < 1002);
   // Small M: 16 x 16 blocks while they are few (c2's shapes: 64x1536x512 4.9
   // against 5.3 us), ring tiles (same bits) where the blocks' operand reads
@@ -1305,29 +1266,19 @@ static int launch_gemm_typed(const GemmArgs& g0, hipStream_t st) {
   }
   const bool big_ok = g.k % 64 == 0 && g.m >= 256 && vec_ok;
   if (!big_ok || variant == 0) return launch_gemm_small<T, TC, TB, TR, QKV>(g, st);
-  // fp32 C with short K: gemm_hp_kernel's staged epilogue covers 16-bit C
-  // only, and its direct fp32 epilogue on 256-wide tiles took 471 us at
-  // 100000x1024x1024, where ring tiles take 360.
-  // Tall operands (M >= 32768, so A streams from HBM rather than staying in
-  // the caches) with a short K panel (K <= 2048): of the 256-row tiles the
-  // 128-wide ones, whose third K stage covers the longer latency; ring tiles
-  // of 128 x 192 where the model prefers them (100000 rows: QKV 663 -> 612
-  // us, FFN-in 1058 -> 971).
-  const bool tall = g.m >= 32768 && g.k <= 2048;
   if (variant < 0) {
-    double hp_us = 0.0;
-    const bool big128 = !tall && sizeof(TC) == 4 && !(g.epi & TX_EPI_SPLIT_OUT) && g.k < 4096;
-    variant = tall ? 128 : hp_width(g, cus);
-    hp_us = hp_model_us(g, cus, variant);
-    // gemm_hp_kernel writes V^T element by element when a 16-row chunk can
-    // span two sequences; gemm_ring_kernel does not (S = 421, 2105x3072x1024:
-    // 24.3 against 21.2 us, where the model has 19.6 and 20.7).
-    if (QKV && g.seq % 16 != 0) hp_us *= 1.2;
-    if (big128) variant = 20;
-    // Smaller tiles where their modelled time is less (ring_pick), and for
-    // all fp32 results that took the 128x128 kernel (16000x1024x1024 53 to 55
-    // against 56 us, 5003x1024x1024 20 against 26 us).
-    if (ring_ok && (big128 || ring_us < hp_us)) return ring(ring_cfg, false);
+    GemmShape s{};
+    s.m = g.m;
+    s.n = g.n;
+    s.k = g.k;
+    s.gelu = g.epi & TX_EPI_GELU_ERF;
+    s.residual = g.epi & TX_EPI_RESIDUAL;
+    s.split = !QKV && (g.epi & TX_EPI_SPLIT_OUT);
+    s.f32 = sizeof(TC) == 4 && !s.split;
+    s.qkv = QKV;
+    s.seq = g.seq;
+    variant = gemm_route(s, cus, ring_ok);
+    if (variant >= 1000) return ring(variant - 1000, false);
   }
   // gemm_hp_kernel's per-lane DMA offsets are 32-bit (hp_offsets_fit); wider
   // row strides take the 128x128 kernel, which addresses in 64 bits.

@@ -384,49 +384,6 @@ static int launch_cfg(const GemmArgs& g0, hipStream_t st) {
   return hipGetLastError() == hipSuccess ? TX_OK : TX_EHIP;
 }
 
-// Tile configurations: BM, BN, workgroups resident per CU (LDS stages in
-// launch_typed), and the launch time's model
-//   t = c + rounds (a k + e + gelu g),
-// rounds of at most `per_cu` tiles a CU; a last round of at most one tile a
-// CU runs at its own rate (a1, e1, g / 2).  Least squares over 290 random
-// shapes (M 257 .. 20000, N and K the projections and MLPs of d_model 256 ..
-// 2048, operands rotated through six sets; standard error 6-10%),
-// microseconds.  Picking the least modelled time is 1-3% off the best
-// configuration of each shape, and against the 256-row tiles alone 1.65 times
-// the speed up to M = 12000 (geometric mean; at M = 1024, N = 512, K = 2048: 28 ->
-// 9.4 us) and 1.07 times over M 2600 .. 20000 at d_model 1024 and 2048.
-struct RingCfg {
-  int bm, bn, per_cu;
-  double c, a, e, g, a1, e1;
-};
-static const RingCfg RING[] = {
-    {64, 64, 2, 2.76, 0.00568, 1.73, 0.613, 0.00356, 0.965},
-    {64, 128, 1, 1.69, 0.00484, 2.54, 1.05, 0.00484, 2.54},
-    {128, 128, 1, 0.967, 0.00727, 4.27, 2.16, 0.00727, 4.27},
-    {128, 128, 2, 2.48, 0.0144, 3.43, 3.47, 0.0108, 1.82},
-    {128, 192, 1, 0.0, 0.00923, 6.13, 3.27, 0.00923, 6.13},
-    {128, 192, 2, 2.43, 0.0185, 5.66, 5.3, 0.0121, 2.94},
-};
-
-// The configuration of least modelled time for the shape (us in *cost); ks4:
-// of those that have the four-sum order.
-int ring_pick(int m, int n, int k, bool gelu, int cus, bool ks4, double* cost) {
-  int best = 0;
-  for (int c = 0; c < (ks4 ? 2 : (int)(sizeof(RING) / sizeof(RING[0]))); ++c) {
-    const RingCfg& r = RING[c];
-    const long tiles = (long)((m + r.bm - 1) / r.bm) * ((n + r.bn - 1) / r.bn), slots = (long)cus * r.per_cu;
-    const long full = tiles / slots, rem = tiles - full * slots;
-    const double g = gelu ? r.g : 0.0;
-    double t = r.c + (double)full * (r.a * k + r.e + g);
-    if (rem > 0) t += rem <= cus ? r.a1 * k + r.e1 + g / r.per_cu : r.a * k + r.e + g;
-    if (c == 0 || t < *cost) {
-      best = c;
-      *cost = t;
-    }
-  }
-  return best;
-}
-
 template <typename T, typename TC, typename TR, bool QKV>
 static int launch_typed(const GemmArgs& g, int cfg, bool ks4, hipStream_t st) {
   switch (cfg) {

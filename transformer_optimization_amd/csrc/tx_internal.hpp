@@ -75,9 +75,8 @@ struct AttnArgs {
 int launch_layernorm(const LayerNormArgs& a, hipStream_t st);
 int launch_gemm(const GemmArgs& g, int ab_dt, int c_dt, int bias_dt, int res_dt, bool qkv,
                 hipStream_t st);
-// gemm_ring.hip (K a multiple of 64, vector-aligned C, 32-bit tile offsets):
-// the tile configuration of least modelled time, and its launch.
-int ring_pick(int m, int n, int k, bool gelu, int cus, bool ks4, double* cost_us);
+// gemm_ring.hip (K a multiple of 64, vector-aligned C, 32-bit tile offsets): the
+// launch of tile configuration cfg (gemm_route.hpp).
 int launch_gemm_ring(const GemmArgs& g, int ab_dt, int c_dt, int res_dt, bool qkv, int cfg, bool ks4,
                      hipStream_t st);
 int launch_attention(const AttnArgs& a, int dt, hipStream_t st);
