@@ -115,18 +115,18 @@ inline int gemm_route(const GemmShape& s, int cus, bool ring_ok) {
   const double ragged = s.qkv && s.seq % 16 != 0 ? 1.2 : 1.0;
   // Tall operands (A streams from HBM rather than staying in the caches) with a
   // short K panel: of the 256-row tiles the 128-wide ones, whose third K stage
-  // covers the longer latency.  Such launches are bound by memory more than the
-  // fitted ones were, which costs the 128 x 128 ring tiles most (less beside a
-  // GELU) and the 128 x 192 ones where the epilogue writes four bytes an
-  // element without reading a residual; the factors are what 321 random calls
-  // with M 32768 .. 131072 asked for.  Against the 256-row tiles alone they take
-  // 0.948 of the time (geometric mean), the uncorrected model 0.954 with calls up to
-  // 1.12 times as long (us, 256-row / 128x128 / 128x192: fp32 35138x768x768
-  // 75 / 75 / 84, fp32 121852x1024x1024 368 / 398 / 370, pairs 107795x2048x512 533 /
-  // 500 / 580, 16-bit 130663x1024x1024 345 / 363 / 342).
+  // covers the longer latency.  The fit ends at 20000 rows; here, relative to
+  // the 256-row tiles, the 128 x 128 ring tiles take longer than modelled except
+  // beside a GELU and for pairs, and the 128 x 192 ones where the epilogue writes
+  // four bytes an element without reading a residual.  The factors come from 321
+  // random calls with M 32768 .. 131072: 0.947 of the time of the 256-row tiles
+  // alone (geometric mean; 7 calls over 1.03, the longest 1.06), without them
+  // 0.954 (42 calls over 1.03, the longest 1.12).  In us, 256-row / 128x128 /
+  // 128x192: fp32 35138x768x768 75 / 75 / 84, fp32 121852x1024x1024 368 / 398 / 370,
+  // pairs 107795x2048x512 533 / 500 / 580, 16-bit 130663x1024x1024 345 / 363 / 342.
   if (s.m >= 32768 && s.k <= 2048) {
     const double hp = gemm_hp_us(128, s.m, s.n, s.k, s.gelu, cus) * ragged;
-    const double r128 = gemm_ring_us(3, s.m, s.n, s.k, s.gelu, cus) * (s.gelu ? 1.0 : 1.15);
+    const double r128 = gemm_ring_us(3, s.m, s.n, s.k, s.gelu, cus) * (s.split ? 0.95 : s.gelu ? 1.0 : 1.15);
     const double r192 = gemm_ring_us(5, s.m, s.n, s.k, s.gelu, cus) * (s.gelu || s.qkv ? 1.0 : 1.03);
     const bool no192 = s.split || (s.f32 && !s.residual);
     if (!ring_ok || hp <= (no192 || r128 < r192 ? r128 : r192)) return 128;
