@@ -1903,7 +1903,8 @@ static int launch_exact_hd(const AttnArgs& a, dim3 grid, hipStream_t st) {
     //   head dim 128: up to 256 keys four, causal any (64 x 16 x 256 137 / 156,
     //   causal 138 / 131); up to 512 one, causal two (8 x 8 x 512 46.4 / 40.0, 16
     //   x 8 x 512 67.8 / 72.6, causal 51.9 / 50.3); up to 1024 one (2 x 16 x 1000
-    //   79.7 / 68.8), half of one for full rows of natural V (78 / 101).
+    //   79.7 / 68.8), half of one for full rows of natural V (78 / 101: its 82,944
+    //   bytes of LDS leave room for one workgroup per CU).
     // tx_select_kernel forces either path (tests and timing).
     const int forced = selected_kernel(TX_SELECT_ATTN_ROWRES);
     const long cus = device_cu_count() > 0 ? device_cu_count() : 256;

@@ -1,14 +1,19 @@
-// gemm_ring_kernel: GEMMs whose output has too few 256-row tiles to fill the
-// CUs (the reference CLI's default shape, B8 S128 D512 F2048, gives
-// gemm_hp_kernel 16 to 64 tiles on 256 CUs).
+// gemm_ring_kernel: tiles of 64 to 128 rows.  First of all for outputs with too
+// few 256-row tiles to fill the CUs (the reference CLI's default shape, B8 S128
+// D512 F2048, gives gemm_hp_kernel 16 to 64 tiles on 256 CUs), and for any other
+// whose modelled time is less (gemm_route.hpp), up to 100000 rows.
 //
-// One workgroup of eight waves (2 x 4) per BM x BN tile (64 to 128 rows, 64 to
-// 192 columns), not persistent: with two workgroups per CU one's epilogue and
-// first loads run beside the other's K loop.  K advances in steps of 64 through NS LDS stages
-// fed by global_load_lds_dwordx4.  A CU pulls about 50 bytes per clock from
-// L2 at a latency of 800 ns and more (weights inside a forward come from HBM
-// or the MALL), so what bounds these shapes is the bytes in flight per CU:
-// the ring is as deep as LDS allows.
+// One workgroup of eight waves (2 x 4) per BM x BN tile (64 to 192 columns), not
+// persistent: with two workgroups per CU one's epilogue and first loads run
+// beside the other's K loop.  K advances in steps of 64 through NS LDS stages
+// fed by global_load_lds_dwordx4.
+//
+// What bounds it: at few tiles waits (waves wait half of their life at 1024 rows,
+// vector and matrix pipes both far from busy): the first loads, the LDS port in
+// the K step (a 64 x 64 step moves 48 KB of fragments and 16 KB of DMA; eight
+// stages instead of four took 9.6 against 9.3 us at 1024x512x2048, so it is not
+// the bytes in flight), and CUs without a tile.  On full grids the matrix cores
+// are 0.3 to 0.42 busy and, with GELU, the vector ALUs 0.38 to 0.52.
 //
 // Inside a step, as in gemm_hp_kernel: the MFMAs (v_mfma_f32_16x16x32) of
 // k32 group 0 with the fragment reads of group 1 between them; the wait for
@@ -311,7 +316,7 @@ __global__ __launch_bounds__(512) void gemm_ring_kernel(GemmArgs g) {
         }
         __syncthreads();
         // V^T rows: per column, the tile's rows are up to two runs of sequence
-        // positions (stage16 & 2: seq >= BM), each written as 8-position
+        // positions (staged only where seq >= BM), each written as 8-position
         // chunks aligned in the row; partial chunks element by element.
         const int b0 = m0 / g.seq, s0 = m0 - b0 * g.seq;
         const int rows = min(BM, g.m - m0);

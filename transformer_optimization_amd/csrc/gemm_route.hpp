@@ -63,9 +63,12 @@ inline int gemm_ring_pick(int m, int n, int k, bool gelu, int cus, bool ks4, dou
 // 128 (per-FLOP cost of the narrower wave tiles).  Fitted to every c3/c4
 // GEMM shape with all three widths timed in one process and checked on
 // whole forwards: it picks 256 for c3's FFN-in and c4's out_proj, FFN-in and
-// FFN-out, 192 for the QKV projections, 128 for c3's out_proj and FFN-out.
-// (At c4's QKV the 256-wide tiles win in isolation, 172 vs 181 us, but not
-// inside the forward, where their two K stages see cold operands.)
+// FFN-out, 128 for c3's out_proj and FFN-out.  (192 for the c3 and c4 QKV
+// projections, which take 128 x 192 ring tiles now; at c4's the 256-wide tiles won
+// in isolation, 172 vs 181 us, but not inside the forward, where their two K
+// stages see cold operands.)  gemm_hp_us below does not always agree with it:
+// 4096x4096x1024 with GELU is 128 here and modelled 40.6 us at 256 against 46.0
+// at 128; which is right has not been measured.
 inline int gemm_hp_width(int m, int n, int k, int cus) {
   static const int bn[3] = {256, 192, 128};
   static const double w[3] = {0.97, 1.0, 1.2};
@@ -110,8 +113,12 @@ struct GemmShape {
 // gemm_big_kernel.  ring_ok: gemm_ring_kernel takes the operands.
 inline int gemm_route(const GemmShape& s, int cus, bool ring_ok) {
   // gemm_hp_kernel writes V^T element by element when a 16-row chunk can span
-  // two sequences; gemm_ring_kernel does not (S = 421, 2105x3072x1024: 24.3
-  // against 21.2 us, where the model has 19.6 and 20.7).
+  // two sequences; gemm_ring_kernel does not.  Sequences of 421 to 1645 against
+  // ones of whole 16 rows and nearly the same length, d_model 512, 1024, 2048: the
+  // 256-row tiles take 1.08 to 1.8 times as long, ring tiles 1.04 to 1.4
+  // (2105x3072x1024 24.4 us on 128-wide tiles and 21.9 on ring tiles, modelled
+  // 19.6 and 20.7).  With 1.2 eight of the nine are within 2% of their best kernel;
+  // 2105x6144x2048 takes 78 us on 256-wide tiles, 63 on ring tiles.
   const double ragged = s.qkv && s.seq % 16 != 0 ? 1.2 : 1.0;
   // Tall operands (A streams from HBM rather than staying in the caches) with a
   // short K panel: of the 256-row tiles the 128-wide ones, whose third K stage

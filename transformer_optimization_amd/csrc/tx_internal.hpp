@@ -45,7 +45,9 @@ struct GemmArgs {
   int heads;
   int head_dim;
   int group;  // tile rows per band of the tile order (set by launch_gemm)
-  int stage16;  // 1: gemm_hp_kernel's 16-byte staged epilogue (set by launch_hp)
+  // 1: 16-byte staged epilogue; 2 (gemm_hp_kernel only): V^T columns staged too.
+  // Set by launch_hp and gemm_ring.hip's launch_cfg.
+  int stage16;
 };
 
 // Attention operands as strided [batch, head, seq, head_dim] views (element
